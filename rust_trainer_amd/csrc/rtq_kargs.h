@@ -111,6 +111,27 @@ struct DenseArgs {
   const int32_t* idx;  // or null: out row i is weight row idx[i] (embedding gather), else r0 + i
 };
 
+// rtq_dense_fwd* / rtq_dense_bwd*: y = x W^T or dx = dy W of a trainer-native weight on split bf16 MFMAs
+struct DenseGemmArgs {
+  const float* x;     // the token-side operand: x [T][K] (forward), dy [T][N] (backward)
+  const float* w;     // F32 weight [N][K], or null
+  const float* sc;    // TQ8_0 scales [N][K / 32], or null
+  const int8_t* qs;   // TQ8_0 codes [N][K]
+  int T, N, K;        // K % 32 == 0
+  int nsplit, n_per_split;  // backward: splits of W's rows (n_per_split a multiple of 32); forward: 1, -
+  float* out;         // y [T][N]; partials [nsplit][T][K], or dx
+  int accumulate;     // backward, one split: out += (FrozenMatmul::backward_input)
+  const float* bias;  // forward: [N] or null
+  const float* hp;    // LoRA: forward: slice partials [T][r][nhp] of x A^T, or null; backward, as DxArgs:
+  int nhp;            //   the last workgroups sum hp (nhq slices) and gp (ngq) to h and g
+  const float* lb;    // forward: B [N][r]; backward: A [r][K]
+  const float* gp;
+  int nhq, ngq, r;
+  float s;
+  float* h;
+  float* g;
+};
+
 // ---------------------------------------------------------------- forward GEMM
 // y[t][n] = sum_b d_w[n][b] d_x[t][b] isum_b(t, n)  (+ bias[n]) (+ s * sum_j h[t][j] B[n][j])
 // K-quants: sum over super-blocks of (d d_x) S1 - (dmin d_x) S2 (Q4_K) or (d d_x) S (Q6_K)
@@ -264,6 +285,7 @@ struct LoraGradArgs {
   float* swdu;
   int64_t swld;
   int sw_keep;  // 1: dh is stored to dx as well (a layer whose activations are being captured)
+  int has_ga;   // 1: the (row-major) partials hold g . A already
 };
 
 // dA / dB of up to RTQ_LORA_JOBS linears in one launch (rtq_lora_grads[16]): workgroups

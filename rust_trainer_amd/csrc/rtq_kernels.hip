@@ -2753,7 +2753,8 @@ struct DxSlot<FMT_Q6_K, NQ> : DxSlot<FMT_Q4_K, NQ> {};
 
 // h = sum of hp, g = s * sum of gp, both in slice order (src/linear.rs:106-111), by the nfin
 // finaliser workgroups of a dx grid (rel: this workgroup's index among them)
-__device__ __forceinline__ void dx_lora_sums(const DxArgs& a, int rel, int nfin) {
+template <class Args>  // DxArgs, DenseGemmArgs
+__device__ __forceinline__ void dx_lora_sums(const Args& a, int rel, int nfin) {
   const int64_t n = (int64_t)a.T * a.r;
   const int64_t nthr = (int64_t)nfin * blockDim.x;
   for (int64_t e = (int64_t)rel * blockDim.x + threadIdx.x; e < n; e += nthr) {
@@ -3846,7 +3847,7 @@ __device__ __forceinline__ void lora_grad_tile(const LoraGradArgs& a, int b, flo
 // dx[t, k0 .. k0+3] from its summed partials: + g[t] . A[:, k0 .. k0+3] (src/linear.rs:115-118),
 // then stored / accumulated, or (sw) taken as SwiGLU's dh (accumulate is off there)
 __device__ __forceinline__ void finish_row4(const LoraGradArgs& a, int t, int k0, f4 sum, bool sw) {
-  if (a.g) {
+  if (a.g && !a.has_ga) {
     f4 ga = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int j = 0; j < a.r; j++) {
       const float gv = a.g[(int64_t)t * a.r + j];
@@ -4398,4 +4399,5 @@ extern "C" __global__ __launch_bounds__(256) void rtq_head_norm_bwd(HeadArgs a) 
 }
 
 // ============================================================== decoder block (model-level step)
+#include "rtq_dense.hip"
 #include "rtq_model_kernels.hip"

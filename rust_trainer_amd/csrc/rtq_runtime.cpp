@@ -154,7 +154,9 @@ enum Kid {
   K_LORA_GRADS_T16,
   K_DENSE_ROWS,    // trainer-native weights: rows / dequantisation, bias
   K_DENSE_BIAS,
-  K_HEAD_NORM,   // LM head + cross-entropy (Model::head)
+  K_DENSE_FWD,  // + 2 * (64-token tiles) + TQ8_0: trainer-native products on split bf16 MFMAs
+  K_DENSE_BWD = K_DENSE_FWD + 4,
+  K_HEAD_NORM = K_DENSE_BWD + 4,  // LM head + cross-entropy (Model::head)
   K_HEAD_MAX,
   K_HEAD_SUM,
   K_HEAD_GRAD,
@@ -188,6 +190,8 @@ constexpr const char* kKernelNames[] = {
     "rtq_dx32_q4_0",        "rtq_dx32_q8_0",        "rtq_dx32_q4_k",        "rtq_dx32_q6_k",
     "rtq_bwd_finish",       "rtq_bwd_finish16",     "rtq_bwd_finish_dx",    "rtq_bwd_finish_rows",  "rtq_lora_grads",       "rtq_lora_grads16",     "rtq_lora_grads_t",     "rtq_lora_grads_t16",
     "rtq_dense_rows",       "rtq_dense_bias",
+    "rtq_dense_fwd32",      "rtq_dense_fwd32_q8",   "rtq_dense_fwd64",      "rtq_dense_fwd64_q8",
+    "rtq_dense_bwd32",      "rtq_dense_bwd32_q8",   "rtq_dense_bwd64",      "rtq_dense_bwd64_q8",
     "rtq_head_norm",        "rtq_head_max",         "rtq_head_sum",         "rtq_head_grad",
     "rtq_head_norm_bwd",    "rtq_act_prep8_q8_0",   "rtq_act_prep4_q8_0",
     "rtq_rows_q4_0",        "rtq_rows_q8_0",        "rtq_rows_q4_k",        "rtq_rows_q6_k",
@@ -431,11 +435,43 @@ GemvPlan gemv_plan(const rtq_ctx* c, const rtq_weight* w) {
   return g;
 }
 
+// partial-product slices of the LoRA reductions over n columns (multiple of 4, see sum_partials)
+int64_t lora_slices(int64_t n) { return roundup(cdiv(std::max<int64_t>(n, 1), RTQ_ACT_KQ), 4); }
+
+// trainer-native weights: the split-bf16 kernels (rtq_dense_*) take whole 32-column blocks and operands
+// within the 2 GiB range of their 32-bit buffer offsets; other calls run on the strided f32 GEMM.  There
+// the split kernels won at every size measured (us per call with a rank-8 adapter, GEMM / split):
+// 2048 x 1024 at 1, 300, 1024 tokens forward 59 / 19, 71 / 26, 101 / 39, backward 161 / 18, 233 / 38, 321 /
+// 90; 4096 x 4096 forward 203 / 53, 326 / 105, 518 / 225, backward 339 / 27, 550 / 155, 792 / 325
+bool dense_fast(const rtq_weight* w, int64_t t) {
+  const uint64_t lim = 1ull << 31, N = (uint64_t)w->rows, K = (uint64_t)w->cols;
+  return K % 32 == 0 && (uint64_t)t * N * 4 < lim && (uint64_t)t * K * 4 < lim && N * K * 4 < lim;
+}
+// forward workspace of the strided GEMM: h
+size_t dense_min_bytes(int64_t t, int64_t r) { return (size_t)(t * std::max<int64_t>(r, 0)) * 4 + 2 * 256; }
+// 64-token tiles when they fill the chip twice over, else 32-token tiles (out: outputs per token)
+int dense_tok(const rtq_ctx* c, int64_t out, int64_t t) { return cdiv(out, 64) * cdiv(t, 64) >= 2 * c->cu_count ? 64 : 32; }
+// backward: splits of W's rows, for about two workgroups per CU of at least eight 32-row steps each
+struct DenseBwdPlan {
+  int64_t nsplit, nps;
+  int tok;
+};
+DenseBwdPlan dense_bwd_plan(const rtq_ctx* c, const rtq_weight* w, int64_t t) {
+  DenseBwdPlan p;
+  p.tok = dense_tok(c, w->cols, t);
+  const int64_t steps = cdiv(w->rows, 32), tiles = cdiv(w->cols, 64) * cdiv(t, p.tok);
+  const int64_t want = std::max<int64_t>(1, std::min<int64_t>(cdiv(2 * c->cu_count, tiles), steps / 8));
+  p.nps = cdiv(steps, want) * 32;
+  p.nsplit = cdiv(w->rows, p.nps);
+  return p;
+}
+
 FwdPlan fwd_plan(const rtq_weight* w, int64_t t, int64_t r) {
   FwdPlan p{};
   p.T = t;
   if (is_dense(w->type)) {
-    p.dense_bytes = (size_t)(t * std::max<int64_t>(r, 0)) * 4 + 2 * 256;
+    p.dense_bytes = dense_fast(w, t) ? (size_t)(lora_slices(w->cols) * t * std::max<int64_t>(r, 0)) * 4 + 256
+                                     : dense_min_bytes(t, r);
     return p;
   }
   p.skinny = t <= 16;
@@ -500,17 +536,63 @@ rtq_status dense_gemm(rtq_ctx* c, hipStream_t st, int64_t M, int64_t N, int64_t 
 const float* dense_b(const rtq_weight* w) { return w->type == RTQ_TYPE_F32 ? reinterpret_cast<const float*>(w->wq) : nullptr; }
 const rtq_weight* dense_q8(const rtq_weight* w) { return w->type == RTQ_TYPE_TQ8_0 ? w : nullptr; }
 
+// tokens per g-partial workgroup of rtq_bwd_prep (ngq slices).
+// h partials: 16 tokens per workgroup; g partials: 64 where those workgroups alone give every
+// CU one; else 32 where those give at least half of the CUs one and no CU two (the 32-token
+// form splits each slice's rows over two waves, so twice the workgroups run half the MFMA
+// chain); else 64 where those give at least half of the CUs one; else 16.  Measured per
+// configs[2] call (512 tokens): q|k|v (16 slices, r 48) 8.33 -> 7.46 us at 32; gate|up (24
+// slices, r 32, 384 workgroups at 32) 8.53 -> 9.41, so 64 there
+int prep_gtok(const rtq_ctx* c, int64_t t, int64_t ngq) {
+  if (c->gtok == 16 || c->gtok == 32 || c->gtok == 64) return c->gtok;
+  const int64_t g64 = c->g64_min >= 0 ? c->g64_min : c->cu_count / 2, n64 = cdiv(t, 64) * ngq, n32 = cdiv(t, 32) * ngq;
+  return n64 >= std::max<int64_t>(g64, c->cu_count) ? 64 : (n32 >= g64 && n32 <= c->cu_count) ? 32 : n64 >= g64 ? 64 : 16;
+}
+
+void dense_operands(const rtq_weight* w, const float* x, int64_t t, DenseGemmArgs* a) {
+  a->x = x;
+  a->w = dense_b(w);
+  a->sc = w->type == RTQ_TYPE_TQ8_0 ? w->wsc : nullptr;
+  a->qs = w->type == RTQ_TYPE_TQ8_0 ? reinterpret_cast<const int8_t*>(w->wq) : nullptr;
+  a->T = (int)t;
+  a->N = (int)w->rows;
+  a->K = (int)w->cols;
+}
+
 // y = x W^T (src/frozen.rs:121-122); + bias; + s (x A^T) B^T (src/linear.rs:73-93)
 rtq_status enqueue_forward_dense(rtq_ctx* c, const rtq_weight* w, const float* x, int64_t t, float* y,
                                  const float* bias, const float* la, const float* lb, int64_t r, float s, Arena& ar,
                                  hipStream_t st) {
   const int64_t N = w->rows, K = w->cols;
+  const bool lora = la && lb && r > 0;
+  const int64_t nhp = lora_slices(K);
+  // a caller's workspace (rtq_linear_forward_noalloc_d) too small for the slice partials: the strided GEMM
+  if (dense_fast(w, t) && (!lora || ar.off + (size_t)(nhp * t * r) * 4 + 256 <= ar.cap)) {
+    float* hp = lora ? ar.take<float>((size_t)(nhp * t * r)) : nullptr;
+    if (lora) {  // the slice partials of h = x A^T
+      BwdPrepArgs pa{x, la, (int)K, nullptr, nullptr, (int)N, (int)t, (int)r, hp, (int)nhp, nullptr, 0, nullptr, RankBlocks{}, 0, 64};
+      RTQ_TRY(launch(c, K_BWD_PREP, dim3((unsigned)cdiv(t, 16), (unsigned)nhp), dim3(256), st, pa));
+    }
+    const int tok = dense_tok(c, N, t);
+    DenseGemmArgs ga{};
+    dense_operands(w, x, t, &ga);
+    ga.nsplit = 1;
+    ga.out = y;
+    ga.bias = bias;
+    ga.hp = hp;
+    ga.nhp = (int)nhp;
+    ga.lb = lb;
+    ga.r = (int)r;
+    ga.s = s;
+    return launch(c, K_DENSE_FWD + (tok == 64 ? 2 : 0) + (w->type == RTQ_TYPE_TQ8_0 ? 1 : 0),
+                  dim3((unsigned)roundup(cdiv(N, 64) * cdiv(t, tok), 8)), dim3(256), st, ga);
+  }
   RTQ_TRY(dense_gemm(c, st, t, N, K, x, K, 1, 1.0f, dense_b(w), dense_q8(w), 1, K, y, N, false));
   if (bias) {
     DenseArgs da{nullptr, nullptr, nullptr, N, K, 0, t, y, bias, nullptr};
     RTQ_TRY(launch(c, K_DENSE_BIAS, dim3((unsigned)std::min<int64_t>(cdiv(t * N, 256), 8192)), dim3(256), st, da));
   }
-  if (la && lb && r > 0) {
+  if (lora) {
     float* hh = ar.take<float>((size_t)(t * r));
     if (ar.off > ar.cap) return fail(RTQ_ERR_INVALID, "internal: workspace too small");
     RTQ_TRY(dense_gemm(c, st, t, r, K, x, K, 1, 1.0f, la, nullptr, 1, K, hh, r, false));  // h = x A^T
@@ -525,8 +607,54 @@ rtq_status enqueue_backward_dense(rtq_ctx* c, const rtq_weight* w, const float* 
                                   bool accumulate, const float* x, const float* la, const float* lb, int64_t r,
                                   float s, float* ga, float* gb, Arena& ar, hipStream_t st) {
   const int64_t N = w->rows, K = w->cols;
+  const bool lora = la && lb && r > 0;
+  if (dense_fast(w, t)) {
+    // slice partials of h and g -> split partials of dx, g A in the first (the last workgroups sum h and
+    // g) -> rtq_bwd_finish.  One split writes dx itself and leaves dA / dB to the finish
+    const DenseBwdPlan p = dense_bwd_plan(c, w, t);
+    const int64_t nhq = lora_slices(K), ngq = lora_slices(N);
+    const bool direct = p.nsplit == 1;
+    DenseGemmArgs xa{};
+    dense_operands(w, dy, t, &xa);
+    float* part = direct ? dx : ar.take<float>((size_t)(p.nsplit * t * K));
+    if (lora) {
+      float* hp = ar.take<float>((size_t)(nhq * t * r));
+      float* gp = ar.take<float>((size_t)(ngq * t * r));
+      xa.h = ar.take<float>((size_t)(t * r));
+      xa.g = ar.take<float>((size_t)(t * r));
+      if (ar.off > ar.cap) return fail(RTQ_ERR_INVALID, "internal: workspace too small");
+      BwdPrepArgs pa{x, la, (int)K, dy, lb, (int)N, (int)t, (int)r, hp, (int)nhq, gp, (int)ngq, nullptr, RankBlocks{},
+                     0, prep_gtok(c, t, ngq)};
+      RTQ_TRY(launch(c, K_BWD_PREP, dim3((unsigned)cdiv(t, 16), (unsigned)(nhq + ngq)), dim3(256), st, pa));
+      xa.hp = hp;
+      xa.gp = gp;
+      xa.lb = la;
+      xa.nhq = (int)nhq;
+      xa.ngq = (int)ngq;
+      xa.r = (int)r;
+      xa.s = s;
+    }
+    if (ar.off > ar.cap) return fail(RTQ_ERR_INVALID, "internal: workspace too small");
+    xa.nsplit = (int)p.nsplit;
+    xa.n_per_split = (int)p.nps;
+    xa.out = part;
+    xa.accumulate = direct && accumulate ? 1 : 0;
+    const int64_t nfin = lora ? std::min<int64_t>(64, cdiv(t * r, 512)) : 0;  // LoRA finalisers
+    RTQ_TRY(launch(c, K_DENSE_BWD + (p.tok == 64 ? 2 : 0) + (w->type == RTQ_TYPE_TQ8_0 ? 1 : 0),
+                   dim3((unsigned)(roundup(cdiv(K, 64) * cdiv(t, p.tok) * p.nsplit, 8) + nfin)), dim3(256), st, xa));
+    if (direct && !lora) return RTQ_OK;
+    const int64_t jt = cdiv(r, 16);
+    LoraGradArgs fa{dy, xa.h, xa.g, x, la, (int)t, (int)N, (int)K, (int)r, s, gb, ga, dx, 0, 0, 0, part, (int)p.nsplit,
+                    accumulate ? 1 : 0, 1, RankBlocks{}};
+    fa.n_gb = lora ? (int)(cdiv(N, 64) * jt) : 0;
+    fa.n_ga = lora ? (int)(cdiv(K, 64) * jt) : 0;
+    const int nw = lora && t >= 256 ? 16 : 4;
+    fa.n_dx = direct ? 0 : (int)cdiv(t * cdiv(K, 64), nw);
+    fa.has_ga = 1;
+    return launch(c, nw == 16 ? K_BWD_FINISH16 : K_BWD_FINISH, dim3((unsigned)(fa.n_gb + fa.n_ga + fa.n_dx)), dim3(64 * nw), st, fa);
+  }
   RTQ_TRY(dense_gemm(c, st, t, K, N, dy, N, 1, 1.0f, dense_b(w), dense_q8(w), K, 1, dx, K, accumulate));
-  if (la && lb && r > 0) {
+  if (lora) {
     float* hh = ar.take<float>((size_t)(t * r));
     float* g = ar.take<float>((size_t)(t * r));
     if (ar.off > ar.cap) return fail(RTQ_ERR_INVALID, "internal: workspace too small");
@@ -837,14 +965,14 @@ DxPlan dx_plan(const rtq_ctx* c, const rtq_weight* w, int64_t t) {
   return p;
 }
 
-// partial-product slices of the LoRA reductions over n columns (multiple of 4, see sum_partials)
-int64_t lora_slices(int64_t n) { return roundup(cdiv(std::max<int64_t>(n, 1), RTQ_ACT_KQ), 4); }
-
 // backward workspace: h, g [t x r], their slice partials [t][r][slices], dx split partials
 size_t bwd_ws_bytes(const rtq_ctx* c, const rtq_weight* w, int64_t t, int64_t r) {
   const int64_t n = w->rows, k = w->cols;
-  if (is_dense(w->type)) return (size_t)(2 * t * std::max<int64_t>(r, 0)) * 4 + 3 * 256;
-  const int64_t sl = roundup(cdiv(std::max<int64_t>(n, 1), RTQ_ACT_KQ), 4) + roundup(cdiv(std::max<int64_t>(k, 1), RTQ_ACT_KQ), 4);
+  const int64_t sl = lora_slices(n) + lora_slices(k);
+  if (is_dense(w->type)) {
+    const size_t hg = (size_t)((2 + (dense_fast(w, t) ? sl : 0)) * t * std::max<int64_t>(r, 0)) * 4;
+    return hg + (dense_fast(w, t) ? (size_t)(dense_bwd_plan(c, w, std::max<int64_t>(t, 1)).nsplit * t * k) * 4 : 0) + 6 * 256;
+  }
   return (size_t)((2 + sl) * t * std::max<int64_t>(r, 0)) * 4 + dx_plan(c, w, std::max<int64_t>(t, 1)).part_floats * 4 +
          (size_t)(lora_slices(n) * t) * 4 + 7 * 256;
 }
@@ -889,15 +1017,7 @@ rtq_status enqueue_backward(rtq_ctx* c, const rtq_weight* w, const float* dy, in
   float* dymax = dp.tok16 ? nullptr : ar.take<float>((size_t)(ngq * t));
   if (ar.off > ar.cap) return fail(RTQ_ERR_INVALID, "internal: workspace too small");
   if (lora) {
-    // h partials: 16 tokens per workgroup; g partials: 64 where those workgroups alone give every
-    // CU one; else 32 where those give at least half of the CUs one and no CU two (the 32-token
-    // form splits each slice's rows over two waves, so twice the workgroups run half the MFMA
-    // chain); else 64 where those give at least half of the CUs one; else 16.  Measured per
-    // configs[2] call (512 tokens): q|k|v (16 slices, r 48) 8.33 -> 7.46 us at 32; gate|up (24
-    // slices, r 32, 384 workgroups at 32) 8.53 -> 9.41, so 64 there
-    const int64_t g64 = c->g64_min >= 0 ? c->g64_min : c->cu_count / 2, n64 = cdiv(t, 64) * ngq, n32 = cdiv(t, 32) * ngq;
-    int gtok = n64 >= std::max<int64_t>(g64, c->cu_count) ? 64 : (n32 >= g64 && n32 <= c->cu_count) ? 32 : n64 >= g64 ? 64 : 16;
-    if (c->gtok == 16 || c->gtok == 32 || c->gtok == 64) gtok = c->gtok;
+    const int gtok = prep_gtok(c, t, ngq);
     BwdPrepArgs pa{x, la, K, dy, lb, N, (int)t, (int)r, hp, (int)nhq, gp, (int)ngq, dymax, RankBlocks{},
                    have_h ? (int)nhq : 0, gtok};
     if (rb) pa.rb = *rb;
@@ -1205,6 +1325,8 @@ rtq_status rtq_ctx_reserve(rtq_ctx* c, int64_t max_t, int64_t max_rows, int64_t 
   size_t need = fwd_ws_bytes(fwd_plan(&fake, max_t, max_rank));
   for (int64_t t : {std::min<int64_t>(max_t, 16), max_t})  // both dx paths
     need = std::max(need, bwd_ws_bytes(c, &fake, t, max_rank));
+  fake.type = RTQ_TYPE_F32;
+  need = std::max({need, fwd_ws_bytes(fwd_plan(&fake, max_t, max_rank)), bwd_ws_bytes(c, &fake, max_t, max_rank)});
   RTQ_TRY(ensure_ws(c, need));
   return RTQ_OK;
 }
@@ -1985,7 +2107,7 @@ rtq_status rtq_linear_forward_ws_d(rtq_ctx* c, const rtq_weight* w, const float*
   float s;
   RTQ_TRY(check_lora(lora, &on, &r, &s));
   if (t > 0 && (!x || !y)) return fail(RTQ_ERR_INVALID, "null x/y");
-  const size_t need = fwd_ws_bytes(fwd_plan(w, t, on ? r : 0));
+  const size_t need = is_dense(w->type) ? dense_min_bytes(t, on ? r : 0) : fwd_ws_bytes(fwd_plan(w, t, on ? r : 0));
   if (need > ws_bytes)
     return fail(RTQ_ERR_INVALID, "forward of %lld tokens over %lldx%lld needs %zu bytes of scratch; the maximum is %zu",
                 (long long)t, (long long)w->rows, (long long)w->cols, need, ws_bytes);

@@ -1,0 +1,85 @@
+"""The split-bf16 products of the trainer-native weights (rtq_dense_*) against float64, at the edges of
+their tiles: one token, 31 / 32 / 33 and 64 / 65 tokens, rows that leave a tile or a 32-row step ragged,
+a row count that is no multiple of 4 (scalar dy loads), one 32-column block, enough tiles for the
+64-token form, several row splits.  An f32 dot of n terms is within (n / 2 + 2) 2^-24 of the sum of its
+terms' magnitudes however it is ordered; the products here leave out terms below 2^-24 each, so the
+bound below is (n / 16 + 4) 2^-24 of that sum (a rounding per 32-element step and the split's remainder)."""
+import numpy as np
+import pytest
+
+import oracle as O
+import rust_trainer_amd as rt
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(64, 32, 1), (37, 96, 31), (65, 64, 32), (200, 160, 33), (130, 256, 64), (257, 128, 65), (1030, 2048, 17),
+          (4096, 1024, 600)]
+
+
+def _weight(ctx, kind, n, k):
+    w = O.Rng(1).vec_normal(n * k, 0.02).reshape(n, k)
+    if kind == "f32":
+        return rt.HipFrozen.f32(w, n, k, ctx=ctx), w.astype(np.float64)
+    b = rt.pack_trainer_q8_0(w, n, k)
+    nb = n * k // 32
+    return (rt.HipFrozen(rt.TYPE_TQ8_0, b, n, k, ctx=ctx),
+            (b[:4 * nb].view(np.float32).astype(np.float64)[:, None] * b[4 * nb:].view(np.int8).reshape(nb, 32)).reshape(n, k))
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = rt.Context(0)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("kind", ["f32", "tq8"])
+@pytest.mark.parametrize("n,k,t", SHAPES)
+def test_dense_products(ctx, kind, n, k, t):
+    hw, w = _weight(ctx, kind, n, k)
+    x = O.Rng(2).vec_normal(t * k, 1.0).reshape(t, k)
+    dy = O.Rng(3).vec_normal(t * n, 1.0).reshape(t, n) * np.exp(O.Rng(4).vec_normal(t, 2.0))[:, None].astype(np.float32)
+    a = O.Rng(5).vec_normal(7 * k, 0.05).reshape(7, k)
+    b = O.Rng(6).vec_normal(n * 7, 0.05).reshape(n, 7)
+    lin = rt.Linear("dense", hw, bias=O.Rng(7).vec_normal(n, 0.1))
+    lin.lora = rt.Lora(7, 14.0, a, b)
+    eps = 2.0 ** -24
+    x64, dy64, a64, b64 = (v.astype(np.float64) for v in (x, dy, a, b))
+
+    def close(got, want, size, terms):
+        assert (np.abs(np.asarray(got, np.float64).reshape(want.shape) - want) <= (terms / 16 + 4) * eps * size).all()
+
+    y = lin.forward(x, t)
+    h = x64 @ a64.T
+    size = np.abs(x64) @ np.abs(w.T) + np.abs(lin.bias) + 2 * (np.abs(x64) @ np.abs(a64.T)) @ np.abs(b64.T)
+    close(y, x64 @ w.T + lin.bias + 2 * h @ b64.T, 2 * size, k)
+    dx = lin.backward(x, dy, t)
+    size = np.abs(dy64) @ np.abs(w) + 2 * (np.abs(dy64) @ np.abs(b64)) @ np.abs(a64)
+    close(dx, dy64 @ w + 2 * (dy64 @ b64) @ a64, 2 * size, n)
+    close(lin.lora.ga, 2 * (dy64 @ b64).T @ x64, 2 * 2 * (np.abs(dy64) @ np.abs(b64)).T @ np.abs(x64), n + t)
+    close(lin.lora.gb, 2 * dy64.T @ h, 2 * 2 * np.abs(dy64).T @ (np.abs(x64) @ np.abs(a64.T)), k + t)
+    close(hw.forward(x, t), x64 @ w.T, np.abs(x64) @ np.abs(w.T), k)
+    dx0 = O.Rng(8).vec_normal(t * k, 1.0)
+    dx = dx0.copy()
+    hw.backward_input(dy, t, dx)  # accumulates
+    close(dx, dy64 @ w + dx0.reshape(t, k), np.abs(dy64) @ np.abs(w) + np.abs(dx0.reshape(t, k)), n)
+
+
+@pytest.mark.parametrize("kind", ["f32", "tq8"])
+def test_dense_products_keep_infinities(ctx, kind):
+    """A product with an infinite operand is what f32 sums give, not the NaN of an infinity's split."""
+    n, k, t = 70, 64, 40
+    hw, w = _weight(ctx, kind, n, k)
+    x = O.Rng(2).vec_normal(t * k, 1.0).reshape(t, k)
+    dy = O.Rng(3).vec_normal(t * n, 1.0).reshape(t, n)
+    x[3, 5], x[4, 6], x[5, 7], x[5, 8] = np.inf, np.nan, np.inf, -np.inf
+    dy[7, 69], dy[8, 0] = -np.inf, np.nan
+    y = hw.forward(x, t).reshape(t, n)
+    dx = np.zeros(t * k, np.float32)
+    hw.backward_input(dy, t, dx)
+    with np.errstate(invalid="ignore"):
+        for got, want in ((y, x.astype(np.float64) @ w.T), (dx.reshape(t, k), dy.astype(np.float64) @ w)):
+            assert np.array_equal(np.isnan(got), np.isnan(want))
+            inf = np.isinf(want)
+            assert np.array_equal(got[inf], want[inf].astype(np.float32))
+            assert np.isfinite(got[np.isfinite(want)]).all()
