@@ -241,8 +241,8 @@ struct DxArgs {
   const float* dy;
   int T, N, K;
   int n_per_split;      // rows of W per split (multiple of 32)
-  int nsplit;           // splits: grid = Kc * ceil(T/64) * nsplit workgroups (+ LoRA finalisers)
-  float* part;          // [splits][T][K] partial products
+  int nsplit;           // splits (rtq_dx_* / rtq_dxw_*: of the nrem last tiles)
+  float* part;          // partial products
   // LoRA finalisation by the extra workgroups of the last grid row (when gp != null):
   const float* hp;      // [T][r][nhq] partials from rtq_bwd_prep
   const float* gp;      // [ngq][T][r]
@@ -256,6 +256,7 @@ struct DxArgs {
   int dmq;
   float wsc, wunsc;
   const uint16_t* wdr;  // row-major scales (RTQ_WR_INDEX): rtq_dxv1_*
+  int nfull, nrem;      // rtq_dx_* / rtq_dxw_*: tiles summed whole (a multiple of 8), tiles split over nsplit workgroups
 };
 
 // dx[t][k] = [dx +] sum_s part[s][t][k] [+ sum_j g[t][j] A[j][k]];
@@ -286,6 +287,9 @@ struct LoraGradArgs {
   int64_t swld;
   int sw_keep;  // 1: dh is stored to dx as well (a layer whose activations are being captured)
   int has_ga;   // 1: the (row-major) partials hold g . A already
+  // fragment-order partials: the first nfull tiles of the dx kernel have one, the nrem others nsplit; nsub:
+  // 64-token tiles in a tile (rtq_dxw_*: 4)
+  int nfull, nrem, nsub;
 };
 
 // dA / dB of up to RTQ_LORA_JOBS linears in one launch (rtq_lora_grads[16]): workgroups

@@ -2722,6 +2722,10 @@ extern "C" __global__ __launch_bounds__(256) void rtq_bwd_prep(BwdPrepArgs a) {
 //     product is exact); K-quants: the f32 value of ggml's dequantisation ((d*sc)*u - dmin*m, or
 //     (d*sc)*q) split like dy.  Stored transposed ([k][n]), so a lane reads its B fragment (8
 //     consecutive rows of one column) in 16 bytes.
+// Bound by its three MFMAs per product at large T: rtq_dxw_q8_0, 14336 x 4096 at 2048 tokens, 783 -> 704 us
+// (1.02 PFLOP/s of f16 MFMA; a library f16 matmul reaches 1.15 here) with eight lanes per dy row instead
+// of one (the L1 looks up a line per cycle: a load of 64 different rows held the kernel to it) and
+// conflict-free LDS; rtq_dxw_q6_k, 2560 x 9728 at 6792 tokens, 1461 -> 1204 us.
 // Three f16 MFMAs per product (dh.wh + dl.wh + dh.wl): the missing dl.wl term and the rounding
 // of dl leave a relative error near 2^-21 per product; the partial is scaled back by 2^-e (exact).
 // Weights whose values could reach 2^15 are pre-scaled by 2^-sigma (wsc) and scaled back in the
@@ -2732,8 +2736,10 @@ extern "C" __global__ __launch_bounds__(256) void rtq_bwd_prep(BwdPrepArgs a) {
 // W staging: thread -> half hh = tid/256 (hh 0: elements 4gg..4gg+3 of the block, hh 1:
 // 16+4gg..16+4gg+3), row group rgl, rows 2p, 2p+1, k-group gg and block jb, ordered so the code
 // words a wave loads lie in one 512-byte span; the two rows' scales are adjacent (one load).
-// The converted pair of rows goes to LDS as one 32-bit word per column.  Within a column the
-// 8-row groups are XOR-swizzled by the block index so the four blocks' writes use different banks.
+// The converted pair of rows goes to LDS as one 32-bit word per column.  Column k = 32 jb + .. lies at
+// row k ^ jb (its two low bits), its 8-row units XORed with 2 (k / 8 % 2): the words of a half-wave's
+// store (four blocks, eight row pairs) and the 16-byte reads of a fragment (lanes 0-3, 12-15, 20-23,
+// 24-27 are served together) then meet every bank once.
 
 template <int FMT, int NQ = 1>
 struct DxSlot {
@@ -2745,7 +2751,7 @@ template <int NQ>
 struct DxSlot<FMT_Q4_K, NQ> {
   f4 dy[NQ];
   uint32_t q[2];
-  u4v k;  // sub-block scale words of rows 2p (x: blocks 0, 1; y: 2, 3) and 2p+1 (z, w)
+  uint32_t k[2];  // sub-block scale words of blocks 2 (jb / 2), + 1 of rows 2p, 2p+1
   u2v e;  // super-block (d, dmin) of rows 2p, 2p+1
 };
 template <int NQ>
@@ -2790,17 +2796,26 @@ __device__ __forceinline__ void dq_params(uint32_t d16, uint32_t kw, uint32_t ev
 // (2 x 2 MFMA tiles).  256 (large T): wave (wt, wk) = (w / 2, w % 2) owns 64 tokens x 64 columns
 // (4 x 4 tiles), so each dequantised weight element feeds four times the MFMAs; the partials keep
 // the 64-token fragment order of the TW = 64 kernel.
+// float4 index of split sp's partial of (64-token tile tt, K chunk kc): split 0 of every tile at [tt][kc];
+// splits 1 .. of the nrem split workgroup tiles (rt: index among them; sub: tt's place in its nsub
+// 64-token tiles) behind them
+__device__ __forceinline__ int64_t dx_part_at(int tt, int kc, int Kc, int ntt, int sp, int rt, int nrem, int sub,
+                                              int nsub) {
+  if (sp == 0) return ((int64_t)tt * Kc + kc) * 2048;
+  return ((int64_t)ntt * Kc + ((int64_t)(sp - 1) * nrem + rt) * nsub + sub) * 2048;
+}
+
 template <int FMT, int TW>
 __device__ __forceinline__ void dx_tile(const DxArgs& a) {
-  // Flat grid, XCD-aware: consecutive workgroup ids go to the 8 XCDs in turn, so id % 8 selects
-  // a group of row splits and all (token tile, K chunk) workgroups of a split run on one XCD,
-  // whose L2 then fetches that split's dy slice and W rows once.  The last n_fin workgroups
-  // finalise h and g (LoRA).
+  // Tiles (token group, K chunk), K chunks fastest.  The first a.nfull (whole rounds of the chip) are
+  // summed over every row by one workgroup; the a.nrem left are split over a.nsplit workgroups each, so
+  // that the last round is short.  Flat grid, XCD-aware: consecutive ids go to the 8 XCDs in turn, and
+  // each XCD takes a run of neighbouring tiles (of one split): they share dy rows in its L2.  The last
+  // workgroups finalise h and g (LoRA).
   constexpr int TS = TW == 64 ? 2 : 4, KS = TS;  // MFMA tiles per wave in tokens and in columns
   constexpr int NQ = TW / 64;                     // float4 of dy staged per thread and step
-  const int Kc = a.Kp / 128, ntt = (a.T + 63) / 64, nwt = (a.T + TW - 1) / TW;
-  const int nunit = a.nsplit * nwt;  // (token group, row split) units of Kc workgroups each
-  const int nmain = (nunit + 7) / 8 * 8 * Kc;
+  const int Kc = a.Kp / 128, ntt = (a.T + 63) / 64;
+  const int nrs = a.nrem * a.nsplit, nmain = a.nfull + (nrs + 7) / 8 * 8;  // nfull % 8 == 0
   const int id = blockIdx.x;
   if (id >= nmain) {
     dx_lora_sums(a, id - nmain, gridDim.x - nmain);
@@ -2808,19 +2823,24 @@ __device__ __forceinline__ void dx_tile(const DxArgs& a) {
   }
   constexpr int D = TW == 64 ? 4 : 3;
   __shared__ u4v sA[2][TW / 16][2][64];                               // [buf][tile][hi/lo][lane]
-  __shared__ __attribute__((aligned(16))) _Float16 sW[2][2][128][40];   // [buf][hi/lo][k][n]
+  __shared__ __attribute__((aligned(16))) _Float16 sW[2][2][128][32];   // [buf][hi/lo][k][n], swizzled
   __shared__ float sInv[TW];  // 2^-e (times wunsc) of each token row of the tile
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, li = lane & 15, g = lane >> 4;
   const int wt = TW == 64 ? w >> 2 : w >> 1, wk = TW == 64 ? w & 3 : w & 1;
-  // id -> (XCD id % 8, slot id / 8) -> K chunk slot % Kc of unit u = (slot / Kc) * 8 + XCD: the Kc
-  // workgroups of a unit run back to back on one XCD and share its dy rows in that L2; unit
-  // u = token group * nsplit + split, so an XCD's concurrent units also share weight rows
-  const int kc = (id >> 3) % Kc, u = (id >> 3) / Kc * 8 + (id & 7);
-  if (u >= nunit) return;  // padding of the unit count to a multiple of 8 (uniform, before any barrier)
-  const int sp = u % a.nsplit;
-  const int t0 = (u / a.nsplit) * TW;
-  const int n0 = sp * a.n_per_split;
-  const int nsteps = (min(n0 + a.n_per_split, a.Np) - n0) / 32;
+  int tile, sp = 0, n0 = 0, n_len = a.Np;
+  if (id < a.nfull) {
+    tile = (id & 7) * (a.nfull >> 3) + (id >> 3);
+  } else {
+    const int xcd = id & 7, in = (id - a.nfull) >> 3, per = nrs >> 3, rem = nrs & 7;
+    if (in >= per + (xcd < rem ? 1 : 0)) return;  // padding to a multiple of 8 (uniform, before any barrier)
+    const int q = xcd * per + min(xcd, rem) + in;
+    sp = q / a.nrem;
+    tile = a.nfull + q % a.nrem;
+    n0 = sp * a.n_per_split;
+    n_len = a.n_per_split;
+  }
+  const int kc = tile % Kc, t0 = tile / Kc * TW;
+  const int nsteps = (min(n0 + n_len, a.Np) - n0) / 32;
   const f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
   f4 acc[TS][KS];
 #pragma unroll
@@ -2828,10 +2848,10 @@ __device__ __forceinline__ void dx_tile(const DxArgs& a) {
 #pragma unroll
     for (int j = 0; j < KS; j++) acc[i][j] = zero;
 
-  // dy loader: tokens tl + 64 m (m < NQ), float4 q4 (columns ns + 4 q4 .. +3 of the step); wave w
-  // covers tokens 16 (w % 4) .. +15 and float4 columns 4 (w / 4) .. +3, so its 64 lanes write the
-  // bf16 halves of 32 consecutive A-fragment lanes (512 contiguous bytes: no LDS bank conflicts)
-  const int tl = 16 * ((tid >> 6) & 3) + (tid & 15), q4 = 4 * (tid >> 8) + ((tid >> 4) & 3);
+  // dy loader: tokens tl + 64 m (m < NQ), float4 q4 (columns ns + 4 q4 .. +3 of the step); eight
+  // consecutive lanes take a row's 128 bytes (one or two L1 lines), and a wave's eight rows are 4 apart
+  // (two sets), so that its 8-byte LDS writes at slot (row ^ q4 / 2) + 16 (q4 / 2) meet every bank once
+  const int wv = tid >> 6, tl = 16 * (wv >> 1) + 2 * (wv & 1) + 4 * ((lane >> 3) & 3) + (lane >> 5), q4 = lane & 7;
   const __amdgpu_buffer_rsrc_t rdy = make_rsrc(a.dy, (uint32_t)a.T * a.N * 4u);
   const uint32_t dy_off = ((uint32_t)(t0 + tl) * a.N + 4 * q4) * 4u;
   const bool dy_vec = (a.N & 3) == 0;
@@ -2854,8 +2874,8 @@ __device__ __forceinline__ void dx_tile(const DxArgs& a) {
       q_off[r] = ((((((uint32_t)rgl * Kc + kc) * 2 + (jb >> 1)) * 64 + FL0 + r) * 2 + (jb & 1)) * 2 + hh) * 4u;
   }
   // scales of rows li0, li0+1: adjacent fp16 (Q4_0, Q8_0); for K-quants the two rows' sub-block
-  // words (one 16-byte load) and super-block pairs (one 8-byte load)
-  const uint32_t d_off = KQ ? (uint32_t)RTQ_WR_INDEX(rgl, kc, Kc, li0, 0) * 2u
+  // words and super-block pairs (one 8-byte load)
+  const uint32_t d_off = KQ ? (uint32_t)RTQ_WR_INDEX(rgl, kc, Kc, li0, jb & 2) * 2u
                             : (uint32_t)RTQ_WD_INDEX(rgl, kc, Kc, li0, jb) * 2u;
   const uint32_t e_off = (uint32_t)RTQ_WSB_INDEX(rgl, kc >> 1, Kc >> 1, li0) * 4u;
   const uint32_t q_rg = (uint32_t)Kc * 64 * 16 * (B8 ? 2 : 1);  // bytes per row group
@@ -2869,7 +2889,7 @@ __device__ __forceinline__ void dx_tile(const DxArgs& a) {
   {
     __shared__ float sRed[512];
     constexpr int PER = 512 / TW;
-    const int q0 = n0 / 256, q1 = min((n0 + a.n_per_split + 255) / 256, a.dmq);
+    const int q0 = n0 / 256, q1 = min((n0 + n_len + 255) / 256, a.dmq);
     const int tok = tid % TW, t = t0 + tok;
     float mx = 0.0f;
     if (t < a.T) {
@@ -2913,7 +2933,8 @@ __device__ __forceinline__ void dx_tile(const DxArgs& a) {
 #pragma unroll
     for (int r = 0; r < 2; r++) S.q[r] = __builtin_amdgcn_raw_buffer_load_b32(rq, q_off[r], srg * q_rg, 0);
     if constexpr (KQ) {
-      S.k = __builtin_bit_cast(u4v, __builtin_amdgcn_raw_buffer_load_b128(rd, d_off, srg * d_rg, 0));
+#pragma unroll
+      for (int r = 0; r < 2; r++) S.k[r] = __builtin_amdgcn_raw_buffer_load_b32(rd, d_off + 8u * r, srg * d_rg, 0);
       S.e = __builtin_bit_cast(u2v, __builtin_amdgcn_raw_buffer_load_b64(re, e_off, srg * e_rg, 0));
     } else {
       S.d = __builtin_amdgcn_raw_buffer_load_b32(rd, d_off, srg * d_rg, 0);
@@ -2939,7 +2960,7 @@ __device__ __forceinline__ void dx_tile(const DxArgs& a) {
       const half2v l23 = pk_rtz(fmaf(dv[2], dsc[m], -(float)h23.x), fmaf(dv[3], dsc[m], -(float)h23.y));
       const u2v hv = {__builtin_bit_cast(uint32_t, h01), __builtin_bit_cast(uint32_t, h23)};
       const u2v lv = {__builtin_bit_cast(uint32_t, l01), __builtin_bit_cast(uint32_t, l23)};
-      const int fl = (tl & 15) + 16 * (q4 >> 1);
+      const int fl = ((tl & 15) ^ (q4 >> 1)) + 16 * (q4 >> 1);
       reinterpret_cast<u2v*>(&sA[buf][(tl >> 4) + 4 * m][0][fl])[q4 & 1] = hv;
       reinterpret_cast<u2v*>(&sA[buf][(tl >> 4) + 4 * m][1][fl])[q4 & 1] = lv;
     }
@@ -2950,7 +2971,7 @@ __device__ __forceinline__ void dx_tile(const DxArgs& a) {
 #pragma unroll
       for (int r = 0; r < 2; r++) {
         float d, m;
-        dq_params<FMT>(0u, comp(S.k, 2 * r + (jb >> 1)), r ? S.e.y : S.e.x, jb, hh, d, m);
+        dq_params<FMT>(0u, S.k[r], r ? S.e.y : S.e.x, jb, hh, d, m);
         d *= a.wsc;  // exact (a power of two; 1 unless a scale is huge)
         m *= a.wsc;
         const uint32_t u = B8 ? S.q[r] ^ 0x80808080u : (hh ? (S.q[r] >> 4) : S.q[r]) & 0x0f0f0f0fu;
@@ -2983,11 +3004,11 @@ __device__ __forceinline__ void dx_tile(const DxArgs& a) {
       }
     }
     const int kb = 32 * jb + 16 * hh + 4 * wgg;
-    const int ns = nloc ^ (8 * jb);  // swizzled row (pair start stays even)
+    const int ns = nloc ^ (16 * ((kb >> 3) & 1));  // 16-byte unit n / 8, XORed with 2 (k / 8 % 2)
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-      *reinterpret_cast<uint32_t*>(&sW[buf][0][kb + e][ns]) = hw[e];
-      *reinterpret_cast<uint32_t*>(&sW[buf][1][kb + e][ns]) = lw[e];
+      *reinterpret_cast<uint32_t*>(&sW[buf][0][kb + (e ^ jb)][ns]) = hw[e];
+      *reinterpret_cast<uint32_t*>(&sW[buf][1][kb + (e ^ jb)][ns]) = lw[e];
     }
   };
   // the wave's operand fragments of one step: A (dy) hi / lo of its two token tiles, B (W) hi / lo
@@ -2995,18 +3016,19 @@ __device__ __forceinline__ void dx_tile(const DxArgs& a) {
   struct Frags {
     half8 a[TS][2], b[KS][2];
   };
+  const int asl = (li ^ g) + 16 * g;
   auto load_frags = [&](int buf, Frags& F) {
 #pragma unroll
     for (int ts = 0; ts < TS; ts++) {
-      F.a[ts][0] = __builtin_bit_cast(half8, sA[buf][wt * TS + ts][0][lane]);
-      F.a[ts][1] = __builtin_bit_cast(half8, sA[buf][wt * TS + ts][1][lane]);
+      F.a[ts][0] = __builtin_bit_cast(half8, sA[buf][wt * TS + ts][0][asl]);
+      F.a[ts][1] = __builtin_bit_cast(half8, sA[buf][wt * TS + ts][1][asl]);
     }
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
-      // column kl lies in block kl / 32, whose rows are swizzled by 8 (kl / 32)
-      const int kl = wk * 16 * KS + ks * 16 + li, jbk = (wk * 16 * KS + ks * 16) >> 5;
-      F.b[ks][0] = *reinterpret_cast<const half8*>(&sW[buf][0][kl][8 * (g ^ jbk)]);
-      F.b[ks][1] = *reinterpret_cast<const half8*>(&sW[buf][1][kl][8 * (g ^ jbk)]);
+      // column k0 + li lies in block k0 / 32: row (k0 + li) ^ (k0 / 32), unit g ^ 2 (li / 8)
+      const int k0 = wk * 16 * KS + ks * 16, kl = k0 + (li ^ (k0 >> 5)), ul = 8 * (g ^ (2 * (li >> 3)));
+      F.b[ks][0] = *reinterpret_cast<const half8*>(&sW[buf][0][kl][ul]);
+      F.b[ks][1] = *reinterpret_cast<const half8*>(&sW[buf][1][kl][ul]);
     }
   };
   auto compute = [&](const Frags& F) {
@@ -3065,12 +3087,13 @@ __device__ __forceinline__ void dx_tile(const DxArgs& a) {
 #pragma unroll
       for (int ks = 0; ks < KS; ks++) acc[ts][ks][i] *= sv;
     }
-  // partial tile of this split in fragment order: part[sp][tile][wave][q][lane] (float4 each),
-  // tile = 64-token tile * Kc + K chunk, wave = 4 wt' + wk', q = 2 ts' + ks' in the TW = 64 layout:
-  // element i is row 64 tile + 32wt' + 16ts' + 4g + i, column 128kc + 32wk' + 16ks' + li.  Each
-  // 16-byte store of a wave writes 1 KB contiguously.
+  // 64-token partial tiles in fragment order, [wave][q][lane] (float4 each), wave = 4 wt' + wk', q = 2 ts'
+  // + ks' in the TW = 64 layout: element i is row 64 tile + 32wt' + 16ts' + 4g + i, column 128kc + 32wk' +
+  // 16ks' + li.  Each 16-byte store of a wave writes 1 KB contiguously.  The first split of every tile at
+  // [64-token tile][K chunk], the others of the nrem split tiles behind them (dx_part_at)
+  f4* part = reinterpret_cast<f4*>(a.part) + lane;
   if (TW == 64) {
-    f4* out = reinterpret_cast<f4*>(a.part) + ((((int64_t)sp * ntt + (t0 >> 6)) * Kc + kc) * 8 + w) * 256 + lane;
+    f4* out = part + dx_part_at(t0 >> 6, kc, Kc, ntt, sp, tile - a.nfull, a.nrem, 0, 1) + w * 256;
 #pragma unroll
     for (int ts = 0; ts < 2; ts++)
 #pragma unroll
@@ -3078,7 +3101,7 @@ __device__ __forceinline__ void dx_tile(const DxArgs& a) {
   } else {
     const int tt64 = (t0 >> 6) + wt;  // this wave's 64 tokens form one 64-token tile
     if (tt64 < ntt) {
-      f4* out = reinterpret_cast<f4*>(a.part) + (((int64_t)sp * ntt + tt64) * Kc + kc) * 8 * 256 + lane;
+      f4* out = part + dx_part_at(tt64, kc, Kc, ntt, sp, tile - a.nfull, a.nrem, wt, 4);
 #pragma unroll
       for (int ts = 0; ts < 4; ts++)
 #pragma unroll
@@ -3919,8 +3942,13 @@ __device__ __forceinline__ void bwd_finish(const LoraGradArgs& a) {
     const int f = fq >> 2, q = fq & 3, ts = q >> 1, ks = q & 1;
     const int tile = f >> 3, dw = f & 7, wt = dw >> 2, wk = dw & 3;
     const int t0 = (tile / Kc) * 64 + wt * 32 + ts * 16, k0 = (tile % Kc) * 128 + wk * 32 + ks * 16;
+    // split 0, and (split tiles) splits 1 .. at p1 + (sp - 1) sstride
+    const int tt = tile / Kc, kc = tile % Kc, wtile = tt / a.nsub * Kc + kc;  // the dx kernel's tile
+    const int nsp = wtile < a.nfull ? 1 : a.nsplit;
     const f4* pp = reinterpret_cast<const f4*>(a.part) + (int64_t)f * 256 + q * 64 + lane;
-    const int64_t sstride = (int64_t)ntt * Kc * 8 * 256;  // f4 per split
+    const int64_t sstride = (int64_t)a.nrem * a.nsub * 2048;
+    const f4* p1 = reinterpret_cast<const f4*>(a.part) + dw * 256 + q * 64 + lane +
+                   dx_part_at(tt, kc, Kc, ntt, 1, wtile - a.nfull, a.nrem, tt % a.nsub, a.nsub);
     const int trow = t0 + li, kcol = k0 + li;
     // g . A operands (f32 MFMA; lane: token 4g + i, column li) of rank chunk jj; the first MAXJ
     // chunks' loads are issued with the partials', so the tile waits for one round of loads
@@ -3953,15 +3981,15 @@ __device__ __forceinline__ void bwd_finish(const LoraGradArgs& a) {
     }
     constexpr int MAXS = DXO ? 4 : NW == 16 ? 8 : 16;  // partials loaded at once; more splits are summed MAXS at a time
     f4 ps = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int c0 = 0; c0 < a.nsplit; c0 += MAXS) {
+    for (int c0 = 0; c0 < nsp; c0 += MAXS) {
       f4 v[MAXS];
 #pragma unroll
       for (int sp = 0; sp < MAXS; sp++)
-        if (c0 + sp < a.nsplit) v[sp] = pp[(int64_t)(c0 + sp) * sstride];
+        if (c0 + sp < nsp) v[sp] = c0 + sp == 0 ? pp[0] : p1[(int64_t)(c0 + sp - 1) * sstride];
       if (c0 == 0) ps = v[0];
 #pragma unroll
       for (int sp = 0; sp < MAXS; sp++)
-        if ((c0 > 0 || sp > 0) && c0 + sp < a.nsplit) ps += v[sp];  // split order
+        if ((c0 > 0 || sp > 0) && c0 + sp < nsp) ps += v[sp];  // split order
     }
     f4 ga = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll

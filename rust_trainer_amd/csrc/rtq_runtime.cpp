@@ -230,7 +230,6 @@ struct rtq_ctx {
   std::vector<hipEvent_t> free_events;
   int dx_splits = 0;  // 0: automatic; RTQ_DX_SPLITS overrides (tuning)
   int gtok = 0;       // g-partial tokens per workgroup: 0 automatic, else 16 / 32 / 64 (RTQ_GTOK)
-  int dx_wpc = 1;     // 64-token dx tiles: row splits for about this many workgroups per CU (RTQ_DX_WPC)
   int dx_wide = -1;   // 256-token dx tiles: -1 automatic, 0 never, 1 for every t > 16 (RTQ_DX_WIDE)
   int dx_32 = 0;      // 32-token dx tiles (RTQ_DX_32): 0 never, 1 with the 64-token plan's splits, 2 with
                       // half of them
@@ -908,47 +907,78 @@ rtq_status enqueue_forward(rtq_ctx* c, const rtq_weight* w, const float* x, int6
 
 // ------------------------------------------------------------------ enqueue: backward
 // dx split plan.
-//   t > 16 (rtq_dx_*): K chunks x 64-token tiles x row splits, about one 8-wave workgroup per CU
-//     (more splits add partial-sum traffic: each split writes and the finish kernel reads a
-//     64-token-padded T x K block);
+//   t > 16: K chunks x 64-token tiles (rtq_dx_*) or 256-token tiles (rtq_dxw_*) x row splits, see dx_cost;
 //   t <= 16 (rtq_dx16_*): K chunks x row splits, about two 4-wave workgroups per CU with at least
 //     four 32-row steps each (partials are T x K floats per split; LM head 151936 x 1024 at T = 16,
 //     one backward call, 64 against 96 splits: Q4_0 58.7 / 62.4 us, Q8_0 64.1 / 65.9, Q4_K 72.7 /
 //     73.7, Q6_K 75.1 / 76.1);
-//   rtq_dxw_*: as the first, with 256-token tiles, where that grid fills the CUs (see dx_plan).
 struct DxPlan {
   int64_t splits, nps;
   bool tok16;
   bool wide;  // rtq_dxw_*: 256-token tiles (each dequantised weight element feeds 4x the MFMAs)
   bool t32;   // rtq_dx32_*: 32-token tiles on four-wave workgroups (same partial layout as rtq_dx_*)
   bool v1;    // rtq_dxv1_*: t == 1 on f32 FMAs (partials as rtq_dx16_*)
+  int64_t nfull, nrem;  // t > 16: tiles summed whole, tiles split over `splits` workgroups
   size_t part_floats;
 };
+// The tiles of a t > 16 plan are summed whole in full rounds of the chip (nfull of them; one 256-token
+// workgroup per CU, or two 64-token ones); the rest are split over `splits` workgroups each.  Kind and splits
+// by the time this model gives (us), fitted to the kernels' times over Q4_0 / Q8_0 / Q4_K / Q6_K weights of
+// 3072 x 1024 to 4096 x 14336 at 37 to 2048 tokens (within 15% of 140 measured plans): a 32-row step of a
+// 256-token workgroup 1.6 after 12 of start-up; of a 64-token one 0.65 alone on its CU, 1.0 beside another
+// (K-quants 0.75, 1.15) after 4; each further partial tile (written, read by the finish) 0.05 / 0.02.
+// Measured, us with the finish, the former rule (64-token tiles unless 256-token ones fill 85% of their
+// rounds) / this one: Q4_K 9728 x 2560 at 37, 256, 1001 tokens 37 / 31, 93 / 61, 337 / 184; Q6_K 2560 x 9728
+// at 100, 1001 53 / 43, 271 / 205; Q8_0 6144 x 4096 at 37 46 / 25
+double dx_cost(const rtq_ctx* c, bool wide, bool kq, int64_t steps, int64_t tiles, int64_t splits, int64_t* nfull) {
+  const int64_t cu = c->cu_count, slots = wide ? cu : 2 * cu;
+  const double start = wide ? 12.0 : 4.0, both = wide ? 1.6 : kq ? 1.15 : 1.0, alone = wide ? 1.6 : kq ? 0.75 : 0.65;
+  *nfull = tiles / slots * slots / 8 * 8;  // whole XCD rounds
+  const int64_t wgs = (tiles - *nfull) * splits, len = cdiv(steps, splits), last = wgs % slots;
+  double us = (double)(*nfull / slots) * (steps * both + start) + (double)(wgs / slots) * (len * both + start);
+  if (last) us += len * (last > cu ? both : alone) + start;
+  return us + (double)((splits - 1) * (tiles - *nfull)) * (wide ? 0.05 : 0.02);
+}
 DxPlan dx_plan(const rtq_ctx* c, const rtq_weight* w, int64_t t) {
   DxPlan p;
   p.tok16 = t <= 16;
   const int64_t Kc = w->Kp / 128, steps = w->Np / 32;
-  // 256-token tiles when their grid fills whole rounds of the CUs (at least 85%) with at least 16
-  // row steps per workgroup; the split count rounds to the nearest whole grid (up to 32 splits)
-  const int64_t per_split = Kc * cdiv(t, 256);
-  const int64_t wsplits = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(32, steps),
-                                                                  (c->cu_count + per_split / 2) / per_split));
-  const int64_t wgrid = roundup(cdiv(t, 256) * wsplits, 8) * Kc;
-  const bool wide_fits = 100 * wgrid >= 85 * cdiv(wgrid, c->cu_count) * c->cu_count && steps / wsplits >= 16;
-  p.wide = !p.tok16 && (c->dx_wide == 1 || (c->dx_wide < 0 && wide_fits));
+  const bool kq = is_kquant(w->type);
+  p.wide = false;
+  p.nfull = 0;
+  int64_t splits = 1;
+  if (!p.tok16) {
+    double best = 1e30;
+    for (int kind = 0; kind < 2; kind++) {
+      const bool wide = kind == 1;
+      if (c->dx_wide >= 0 ? wide != (c->dx_wide == 1) : wide && c->dx_32 > 0) continue;
+      const int64_t tiles = Kc * cdiv(t, wide ? 256 : 64);
+      for (int64_t sp = 1; sp <= (wide ? 32 : 16) && (sp == 1 || cdiv(steps, sp) >= 4); sp++) {
+        int64_t nf;
+        const double us = dx_cost(c, wide, kq, steps, tiles, sp, &nf);
+        if (us < best) {
+          best = us;
+          p.wide = wide;
+          p.nfull = nf;
+          splits = sp;
+        }
+        if (tiles == nf) break;  // nothing to split
+      }
+    }
+  }
   p.t32 = !p.tok16 && !p.wide && c->dx_32 > 0;
-  int64_t splits;
+  const int64_t tiles = Kc * cdiv(t, p.wide ? 256 : 64);
   if (p.tok16)
     splits = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(std::max<int64_t>(steps / 4, 1), 256),
                                                     cdiv(2 * c->cu_count, Kc)));
-  else if (p.wide)
-    splits = wsplits;
-  else
-    splits = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(steps, 16),
-                                                    cdiv(c->dx_wpc * c->cu_count, Kc * cdiv(t, 64))));
   if (p.t32 && c->dx_32 == 2) splits = std::max<int64_t>(1, splits / 2);
-  if (c->dx_splits > 0)
+  if (c->dx_splits > 0) {
     splits = std::min<int64_t>(std::min<int64_t>(steps, p.tok16 ? 256 : (p.wide ? 64 : 16)), c->dx_splits);
+    p.nfull = 0;
+  }
+  if (p.t32) p.nfull = 0;
+  p.nrem = p.tok16 ? 0 : tiles - p.nfull;
+  if (p.nrem == 0 && !p.tok16) splits = 1;
   p.nps = cdiv(steps, splits) * 32;
   p.v1 = t == 1 && c->dxv && (uint64_t)(w->Np / 16) * (w->Kp / 128) * 2048u < (1ull << 32);
   // rtq_dxv1_*: about three four-wave workgroups per CU, each split at least 8 row groups of 16.
@@ -961,7 +991,8 @@ DxPlan dx_plan(const rtq_ctx* c, const rtq_weight* w, int64_t t) {
     p.nps = cdiv(ngr, sv) * 16;
   }
   p.splits = cdiv(w->Np, p.nps);
-  p.part_floats = p.tok16 ? (size_t)(p.splits * t * w->cols) : (size_t)(p.splits * roundup(t, 64) * w->Kp);
+  p.part_floats = p.tok16 ? (size_t)(p.splits * t * w->cols)
+                          : (size_t)(cdiv(t, 64) * Kc + (p.splits - 1) * p.nrem * (p.wide ? 4 : 1)) * 8192;
   return p;
 }
 
@@ -1031,17 +1062,22 @@ rtq_status enqueue_backward(rtq_ctx* c, const rtq_weight* w, const float* dy, in
   }
   DxArgs xa{w->wq, w->wd, w->wsb, (int)w->Np, (int)w->Kp, dy, (int)t, N, K, (int)dp.nps, (int)dp.splits, part,
             lora ? hp : nullptr, lora ? gp : nullptr, (int)nhq, (int)ngq, (int)r, s, h, g, dymax, (int)ngq,
-            w->dx_wsc, w->dx_wunsc, w->wdr};
+            w->dx_wsc, w->dx_wunsc, w->wdr, (int)dp.nfull, (int)dp.nrem};
   const int kid = (dp.v1 ? K_DXV1 : dp.tok16 ? K_DX16 : (dp.wide ? K_DXW : (dp.t32 ? K_DX32 : K_DX))) + fmt_index(w->type);
   set_work(c, w, t, 0, true);
-  // t > 16: (token group, split) units of K-chunk workgroups, padded to a multiple of 8 (XCD order)
+  // t > 16: whole tiles, then split ones, padded to a multiple of 8 (XCD order); rtq_dx32_*: (token group,
+  // split) units of K-chunk workgroups
   const int64_t nmain = dp.tok16 ? (w->Kp / 128) * dp.splits
-                                 : roundup(cdiv(t, dp.wide ? 256 : (dp.t32 ? 32 : 64)) * dp.splits, 8) * (w->Kp / 128);
+                        : dp.t32 ? roundup(cdiv(t, 32) * dp.splits, 8) * (w->Kp / 128)
+                                 : dp.nfull + roundup(dp.nrem * dp.splits, 8);
   const int64_t nfin = lora ? std::min<int64_t>(64, cdiv(t * r, 512)) : 0;  // LoRA finalisers
   RTQ_TRY(launch(c, kid, dim3((unsigned)(nmain + nfin)), dim3(dp.tok16 || dp.t32 ? 256 : 512), st, xa));
   const int64_t jt = cdiv(r, 16);
   LoraGradArgs fa{dy, h, g, x, la, (int)t, N, K, (int)r, s, gb, ga, dx, 0, 0, 0, part, (int)dp.splits, accumulate ? 1 : 0,
                   dp.tok16 ? 1 : 0, RankBlocks{}};
+  fa.nfull = (int)dp.nfull;
+  fa.nrem = (int)dp.nrem;
+  fa.nsub = dp.wide ? 4 : 1;
   if (rb) fa.rb = *rb;  // block-diagonal adapter: dB tiles outside every member's block exit at once
   // dB / dA: one workgroup per 64-row x 16-rank tile; dx: one wave per quarter of a dx fragment (or
   // per token and 64 columns); nw waves per workgroup, 16 when the dA / dB tiles reduce over many tokens
@@ -1051,7 +1087,7 @@ rtq_status enqueue_backward(rtq_ctx* c, const rtq_weight* w, const float* dy, in
   fa.n_dx = dp.tok16 ? (int)cdiv(t * cdiv(K, 64), nw) : (int)cdiv((w->Kp / 128) * cdiv(t, 64) * 32, nw);
   // dx alone: row-major partials of more than 16 splits take a workgroup per (token, 64 columns)
   const bool wide_rows = dp.tok16 && dp.splits > 16;
-  const Kid kdx = dp.splits <= 4 ? K_BWD_FINISH_DX : wide_rows ? K_BWD_FINISH_ROWS : K_BWD_FINISH;
+  const Kid kdx = dp.splits <= 4 || dp.nfull > dp.nrem ? K_BWD_FINISH_DX : wide_rows ? K_BWD_FINISH_ROWS : K_BWD_FINISH;
   const unsigned gdx = wide_rows ? (unsigned)(t * cdiv(K, 64)) : 0;
   if (defer) {  // dA / dB later, in a batch; here the dx partials (+ g.A) alone, 4 waves per workgroup
     *defer->job = fa;
@@ -1253,7 +1289,6 @@ rtq_status rtq_ctx_create(int device, rtq_ctx** out) {
   c->device = device;
   c->cu_count = prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 256;
   if (const char* e = getenv("RTQ_DX_SPLITS")) c->dx_splits = atoi(e);
-  if (const char* e = getenv("RTQ_DX_WPC")) c->dx_wpc = std::min(std::max(atoi(e), 1), 4);
   if (const char* e = getenv("RTQ_GTOK")) c->gtok = atoi(e);
   if (const char* e = getenv("RTQ_DX_WIDE")) c->dx_wide = atoi(e) ? 1 : 0;
   if (const char* e = getenv("RTQ_DX_32")) c->dx_32 = std::min(std::max(atoi(e), 0), 2);
@@ -1323,8 +1358,13 @@ rtq_status rtq_ctx_reserve(rtq_ctx* c, int64_t max_t, int64_t max_rows, int64_t 
   fake.Kp = roundup(max_cols, RTQ_CHUNK_Q);
   fake.type = RTQ_TYPE_Q4_0;
   size_t need = fwd_ws_bytes(fwd_plan(&fake, max_t, max_rank));
-  for (int64_t t : {std::min<int64_t>(max_t, 16), max_t})  // both dx paths
-    need = std::max(need, bwd_ws_bytes(c, &fake, t, max_rank));
+  // the dx plans' split tiles: fewer tokens can need more of them
+  for (int type : {RTQ_TYPE_Q4_0, RTQ_TYPE_Q4_K}) {
+    fake.type = type;
+    const int64_t step = std::max<int64_t>(64, roundup(cdiv(max_t, 1024), 64));
+    for (int64_t t = 64; t < max_t; t += step) need = std::max(need, bwd_ws_bytes(c, &fake, t, max_rank));
+    for (int64_t t : {std::min<int64_t>(max_t, 16), max_t}) need = std::max(need, bwd_ws_bytes(c, &fake, t, max_rank));
+  }
   fake.type = RTQ_TYPE_F32;
   need = std::max({need, fwd_ws_bytes(fwd_plan(&fake, max_t, max_rank)), bwd_ws_bytes(c, &fake, max_t, max_rank)});
   RTQ_TRY(ensure_ws(c, need));
