@@ -224,23 +224,6 @@ __device__ __forceinline__ void skinny_tile(const float* S, int nrows, int lds, 
 // With LoRA, workgroup (x, nq) computes h = x . A^T for its 16 tokens over all of K: per quarter
 // the x and A tiles go through LDS to f32 MFMAs, the next quarter's tiles are loaded into registers
 // while the current one is multiplied, and the four waves' column partials are summed in LDS.
-__device__ __forceinline__ void load_seg(const float* p, bool ok, float v[16]) {
-  if (ok) {
-    const f4* src = reinterpret_cast<const f4*>(p);
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const f4 q = src[i];
-      v[4 * i] = q.x;
-      v[4 * i + 1] = q.y;
-      v[4 * i + 2] = q.z;
-      v[4 * i + 3] = q.w;
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < 16; i++) v[i] = 0.0f;
-  }
-}
-
 // (row n, rank j) lies in a member's block of a block-diagonal adapter (always, for a plain one)
 // (member loops unrolled over the fixed capacity: constant indices keep the struct out of scratch)
 __device__ __forceinline__ bool rb_keep(const RankBlocks& b, int n, int j) {
@@ -285,46 +268,46 @@ __device__ __forceinline__ void rb_span(const RankBlocks& b, int r, int n0, int 
 //   P[t][j] = sum over k in [k0, k0 + 256) of S[t][k] * M[j * ldm + k],  t in [t0, t0 + 16), j < r
 // (h = x . A^T, src/linear.rs:85,106).  Written to out[(t * r + j) * pstride + pidx] (slice index
 // fastest, so a consumer sums a token's partials in slice order with a few wide loads).  Columns
-// beyond kend count as zero.  Thread (row tid / 16, segment tid % 16) holds 16 columns of one row
-// of S and of one rank tile of M.
+// beyond kend count as zero.
 
-// thread (row tl, segment sg)'s 16 values of M's rank row j0 + tl, columns k0 + 16 sg .. (zero past
-// r and kend)
-__device__ __forceinline__ void lora_load_m(const float* M, int ldm, int r, int j0, int k0, int kend, float v[16]) {
-  const int tid = threadIdx.x, jr = j0 + (tid >> 4), kk = k0 + (tid & 15) * 16;
-  load_seg(M + (int64_t)jr * ldm + kk, jr < r && kk + 16 <= kend, v);
-  if (jr < r && kk < kend && kk + 16 > kend) {
+// A 16 x 256 tile in LDS, in float4 units: unit u (columns 4u ..) of row t.  The swizzle lets every lane
+// order used here - a row's units in consecutive lanes, 16 columns per thread, and the MFMA operands'
+// (lane (li, g): unit 16w + 4q + g of row li) - meet every bank once (a 16-byte access serves lanes 0-3,
+// 12-15, 20-23, 24-27 together)
+__device__ __forceinline__ int tile_unit(int t, int u) { return t * 64 + (u & 48) + ((u & 15) ^ t ^ (2 * (u >> 5))); }
+
+// rows j0 + w + 4i (wave w, i < 4) of M, columns k0 + 4 lane .. + 3 (zero past r and kend; kend % 4 = 0)
+__device__ __forceinline__ void lora_load_m(const float* M, int ldm, int r, int j0, int k0, int kend, f4 v[4]) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, k = k0 + 4 * lane;
 #pragma unroll
-    for (int i = 0; i < 16; i++) v[i] = kk + i < kend ? M[(int64_t)jr * ldm + kk + i] : 0.0f;
+  for (int i = 0; i < 4; i++) {
+    const int jr = j0 + w + 4 * i;
+    v[i] = jr < r && k < kend ? *reinterpret_cast<const f4*>(M + (int64_t)jr * ldm + k) : f4{0.0f, 0.0f, 0.0f, 0.0f};
   }
 }
 
-// The product for this thread's S values sv (its row's columns k0 + 16 sg .., zero past T and kend)
-// and the first rank tile's M values mv (lora_load_m at j0 = 0, loaded by the caller so that they
-// travel with its own loads); each next tile's loads are issued before the current one is contracted.
-// NTOK = 8: sx already holds the 8 token rows (and zeros in rows 8 .. 15), sv is not read, and only
-// tokens t0 .. t0 + 7 are written.
+// The product for the S tile in sx (written by the caller, no barrier since; zero past T and kend) and
+// the first rank tile's M values mv (lora_load_m at j0 = 0, loaded by the caller so that they travel with
+// its own loads); each next tile's loads are issued before the current one is contracted.
+// NTOK: tokens t0 .. t0 + NTOK - 1 are written (sx's other rows are zeros).
+// Measured against staging by 16 scalar stores a thread (three LDS cycles in four were conflicts), Q8_0 14336 x
+// 4096, 2048 tokens, r = 64: rtq_act_prep_q8_0 45 -> 33 us (also at 80 VGPRs instead of 184), rtq_bwd_prep 103 -> 88.
 template <int NTOK = 16>
-__device__ __forceinline__ void lora_partial_v(const float* sv, float mv[16], int T, const float* M, int ldm,
-                                               int r, int k0, int kend, int t0, float* out, int pstride, int pidx,
-                                               float* sx, float* sm, float* red) {
-  constexpr int LDX = RTQ_ACT_KQ + 1;
-  const int tid = threadIdx.x, tl = tid >> 4, sg = tid & 15;
-  const int lane = tid & 63, w = tid >> 6, li = lane & 15, g = lane >> 4;
-  if (NTOK == 16) {
-#pragma unroll
-    for (int i = 0; i < 16; i++) sx[tl * LDX + sg * 16 + i] = sv[i];
-  }
+__device__ __forceinline__ void lora_partial_v(f4 mv[4], int T, const float* M, int ldm, int r, int k0, int kend, int t0,
+                                               float* out, int pstride, int pidx, const f4* sx, f4* sm, float* red) {
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, li = lane & 15, g = lane >> 4;
   for (int j0 = 0; j0 < r; j0 += 16) {
 #pragma unroll
-    for (int i = 0; i < 16; i++) sm[tl * LDX + sg * 16 + i] = mv[i];
+    for (int i = 0; i < 4; i++) sm[tile_unit(w + 4 * i, lane)] = mv[i];
     if (j0 + 16 < r) lora_load_m(M, ldm, r, j0 + 16, k0, kend, mv);
     __syncthreads();
     f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int u = 0; u < 16; u++) {
-      const int kl = 64 * w + 4 * u + g;
-      acc = mfma_f32(sx[li * LDX + kl], sm[li * LDX + kl], acc);
+    for (int q = 0; q < 4; q++) {  // wave w: columns 64w ..
+      const int u = tile_unit(li, 16 * w + 4 * q + g);
+      const f4 xv = sx[u], av = sm[u];
+#pragma unroll
+      for (int e = 0; e < 4; e++) acc = mfma_f32(xv[e], av[e], acc);
     }
 #pragma unroll
     for (int i = 0; i < 4; i++) red[w * 256 + (4 * g + i) * 16 + li] = acc[i];
@@ -339,17 +322,19 @@ __device__ __forceinline__ void lora_partial_v(const float* sv, float mv[16], in
 }
 
 __device__ __forceinline__ void lora_partial(const float* S, int T, int ks, const float* M, int ldm, int r, int k0,
-                                             int kend, int t0, float* out, int pstride, int pidx, float* sx,
-                                             float* sm, float* red) {
-  const int tid = threadIdx.x, t = t0 + (tid >> 4), kk = k0 + (tid & 15) * 16;
-  float v[16], mv[16];
-  load_seg(S + (int64_t)t * ks + kk, t < T && kk + 16 <= kend, v);
-  if (t < T && kk < kend && kk + 16 > kend) {  // ragged tail
+                                             int kend, int t0, float* out, int pstride, int pidx, f4* sx, f4* sm,
+                                             float* red) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, k = k0 + 4 * lane;
+  f4 v[4], mv[4];
 #pragma unroll
-    for (int i = 0; i < 16; i++) v[i] = kk + i < kend ? S[(int64_t)t * ks + kk + i] : 0.0f;
+  for (int i = 0; i < 4; i++) {
+    const int t = t0 + w + 4 * i;
+    v[i] = t < T && k < kend ? *reinterpret_cast<const f4*>(S + (int64_t)t * ks + k) : f4{0.0f, 0.0f, 0.0f, 0.0f};
   }
   lora_load_m(M, ldm, r, 0, k0, kend, mv);
-  lora_partial_v(v, mv, T, M, ldm, r, k0, kend, t0, out, pstride, pidx, sx, sm, red);
+#pragma unroll
+  for (int i = 0; i < 4; i++) sx[tile_unit(w + 4 * i, lane)] = v[i];
+  lora_partial_v(mv, T, M, ldm, r, k0, kend, t0, out, pstride, pidx, sx, sm, red);
 }
 
 // LoRA-up input-gradient partial over one 256-row slice q of B (g = dy . B, src/linear.rs:111),
@@ -359,7 +344,8 @@ __device__ __forceinline__ void lora_partial(const float* S, int T, int ks, cons
 // B entries outside rb's blocks count as zero; rank tiles with none inside are written as zeros.
 // B's slice (256 rows x 16 ranks) is staged in LDS once per rank tile and shared by the waves;
 // LDS row n of the slice sits at 16n + 16 (n / 64), so the four lane groups of one MFMA step read
-// four different 16-bank spans.  Each wave holds its dy rows in registers in MFMA operand order:
+// four different 16-bank spans, (TW = 64) its four rank quads XORed with n / 4 % 4, so that the
+// rows written by neighbouring lanes do too (the smaller forms, one workgroup per CU, ran 4% slower so).  Each wave holds its dy rows in registers in MFMA operand order:
 //   TW = 64: wave w owns tokens t0 + 16w .. +15 and all 256 rows; lane (token li, group g) loads
 //            rows 64g .. 64g+63 of the slice (256 contiguous bytes), step u contracts row 64g + u;
 //            no cross-wave reduction;
@@ -449,10 +435,18 @@ __device__ __forceinline__ void lora_up_partial(const BwdPrepArgs& a, int t0, in
     if (cur) {
       const int k = k0 + tid;
       float* dst = sb + 16 * tid + 16 * (tid >> 6);
+      const int x = TW == 64 ? 4 * ((tid >> 2) & 3) : 0;
 #pragma unroll
       for (int i = 0; i < 16; i++) {
         const int j = j0 + i;
-        dst[i] = (k < a.N && j < a.r && rb_keep(a.rb, k, j)) ? bv[i] : 0.0f;
+        bv[i] = (k < a.N && j < a.r && rb_keep(a.rb, k, j)) ? bv[i] : 0.0f;
+      }
+      if (TW == 64) {
+#pragma unroll
+        for (int i = 0; i < 16; i += 4) *reinterpret_cast<f4*>(dst + (i ^ x)) = f4{bv[i], bv[i + 1], bv[i + 2], bv[i + 3]};
+      } else {
+#pragma unroll
+        for (int i = 0; i < 16; i++) dst[i] = bv[i];
       }
     }
     if (j0 + 16 < a.r) {
@@ -462,9 +456,9 @@ __device__ __forceinline__ void lora_up_partial(const BwdPrepArgs& a, int t0, in
     if (cur) {
       __syncthreads();
       if (tok_ok) {
-        const float* sg = sb + 16 * kl0 + 16 * (kl0 >> 6) + li;
+        const float* sg = sb + 16 * kl0 + 16 * (kl0 >> 6);  // kl0 % 16 == 0
 #pragma unroll
-        for (int u = 0; u < NU; u++) acc = mfma_f32(v[u], sg[16 * u], acc);
+        for (int u = 0; u < NU; u++) acc = mfma_f32(v[u], sg[16 * u + (TW == 64 ? li ^ (4 * ((u >> 2) & 3)) : li)], acc);
       }
       if (TW == 16 || (TW == 32 && wh == 1)) {
 #pragma unroll
@@ -526,11 +520,13 @@ __device__ __forceinline__ float rtq_silu_grad(float x) {
   return s * (1.0f + x * (1.0f - s));
 }
 
-template <bool QK>
+// NORM: the RMSNorm input form, a kernel of its own (its rows held whole take 182 VGPRs, which halved the
+// other forms' waves per SIMD)
+template <bool QK, bool NORM>
 __device__ __forceinline__ void act_prep(const ActArgs& a) {
-  constexpr int KQ = RTQ_ACT_KQ, LDX = KQ + 1;
-  __shared__ float sx[16 * LDX];
-  __shared__ float sa[16 * LDX];
+  constexpr int KQ = RTQ_ACT_KQ;
+  __shared__ f4 sx[16 * KQ / 4];
+  __shared__ f4 sa[16 * KQ / 4];
   __shared__ float red[4 * 256];
   const int tid = threadIdx.x, tl = tid >> 4, sg = tid & 15;
   const int t0 = blockIdx.x * 16, t = t0 + tl;
@@ -538,15 +534,17 @@ __device__ __forceinline__ void act_prep(const ActArgs& a) {
   const int k0 = blockIdx.y * KQ;
   {
     const int kk = k0 + sg * 16;  // first column of this thread's segment
-    float v[16], mv[16];
+    const int lane = tid & 63, w = tid >> 6;
+    float v[16];
+    f4 mv[4];
     if (a.A) lora_load_m(a.A, a.K, a.r, 0, k0, a.K, mv);  // uniform; in flight during the activation work
-    if (a.na) {  // uniform: v = RMSNorm rows, in the order of rtq_m_rmsnorm's one-wave rows
+    if constexpr (NORM) {  // v = RMSNorm rows, in the order of rtq_m_rmsnorm's one-wave rows
       // wave w normalises rows t0 + 4w .. t0 + 4w + 3 whole (lane l: float4 columns 4l + 256i, i <
       // K / 256), then writes quarter blockIdx.y of each (x, nh) and passes it through LDS (sx) to
       // the thread layout below; quarters beyond K give zeros.  The 1 / rms is written once.
       // every load issued before any is used: addresses clamped into the rows (no branches between
       // the loads), out-of-range values replaced by zeros afterwards
-      const int lane = tid & 63, w = tid >> 6, nv = a.K / 256, qy = blockIdx.y;
+      const int nv = a.K / 256, qy = blockIdx.y;
       const f4 z4 = {0.0f, 0.0f, 0.0f, 0.0f};
       const bool has_b = a.nb != nullptr;
       const float* pb = has_b ? a.nb : a.na;
@@ -598,25 +596,45 @@ __device__ __forceinline__ void act_prep(const ActArgs& a) {
             }
           }
         if (qy == 0 && lane == 0 && row < a.T) a.ninv[row] = ir;
-#pragma unroll
-        for (int e = 0; e < 4; e++) sx[(4 * w + rr) * LDX + 4 * lane + e] = y[e];
+        sx[tile_unit(4 * w + rr, lane)] = y;
       }
-      __syncthreads();
-#pragma unroll
-      for (int i = 0; i < 16; i++) v[i] = sx[tl * LDX + sg * 16 + i];
     } else if (a.sg) {  // uniform: v = silu(g) * u, written to x for the backward
-      float gv[16], uv[16];
-      load_seg(a.sg + (int64_t)t * a.ldsg + kk, t < a.T && kk < a.K, gv);
-      load_seg(a.su + (int64_t)t * a.ldsg + kk, t < a.T && kk < a.K, uv);
+      // wave w: rows w + 4i, lane l: columns 4l .. (a row's 1 KB in one load)
+      f4 gv[4], uv[4];
 #pragma unroll
-      for (int i = 0; i < 16; i++) v[i] = rtq_silu(gv[i]) * uv[i];
-      if (t < a.T && kk < a.K) {
-        f4* xo = reinterpret_cast<f4*>(const_cast<float*>(a.x) + (int64_t)t * a.K + kk);
+      for (int i = 0; i < 4; i++) {
+        const int64_t o = (int64_t)min(t0 + w + 4 * i, a.T - 1) * a.ldsg + min(k0 + 4 * lane, a.K - 4);
+        gv[i] = *reinterpret_cast<const f4*>(a.sg + o);
+        uv[i] = *reinterpret_cast<const f4*>(a.su + o);
+      }
 #pragma unroll
-        for (int i = 0; i < 4; i++) xo[i] = f4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
+      for (int i = 0; i < 4; i++) {
+        const int row = t0 + w + 4 * i;
+        f4 x4 = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (row < a.T && k0 + 4 * lane < a.K) {
+#pragma unroll
+          for (int e = 0; e < 4; e++) x4[e] = rtq_silu(gv[i][e]) * uv[i][e];
+          *reinterpret_cast<f4*>(const_cast<float*>(a.x) + (int64_t)row * a.K + k0 + 4 * lane) = x4;
+        }
+        sx[tile_unit(w + 4 * i, lane)] = x4;
       }
     } else {
-      load_seg(a.x + (int64_t)t * a.K + kk, t < a.T && kk < a.K, v);  // K % 32 == 0: all in or all out
+      f4 xv[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int row = t0 + w + 4 * i;
+        xv[i] = row < a.T && k0 + 4 * lane < a.K ? *reinterpret_cast<const f4*>(a.x + (int64_t)row * a.K + k0 + 4 * lane)
+                                                 : f4{0.0f, 0.0f, 0.0f, 0.0f};
+      }
+#pragma unroll
+      for (int i = 0; i < 4; i++) sx[tile_unit(w + 4 * i, lane)] = xv[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; i++) {  // K % 32 == 0: a thread's 16 columns are all in or all out
+      const f4 x4 = sx[tile_unit(tl, 4 * sg + i)];
+#pragma unroll
+      for (int e = 0; e < 4; e++) v[4 * i + e] = x4[e];
     }
     _Float16 q[16];  // codes: exact small integers
     float dstore;    // the block scale as the dot products use it
@@ -700,7 +718,7 @@ __device__ __forceinline__ void act_prep(const ActArgs& a) {
     // LoRA-down partial of these columns from the values in registers (zero past T and K, like the
     // codes; quarters beyond K write zero partials)
     if (a.A)  // uniform
-      lora_partial_v(v, mv, a.T, a.A, a.K, a.r, k0, a.K, t0, a.hp, gridDim.y, blockIdx.y, sx, sa, red);
+      lora_partial_v(mv, a.T, a.A, a.K, a.r, k0, a.K, t0, a.hp, gridDim.y, blockIdx.y, sx, sa, red);
   }
   if (a.zero_y && blockIdx.y == 0) {
     for (int tt = 0; tt < 16; tt++) {
@@ -711,8 +729,10 @@ __device__ __forceinline__ void act_prep(const ActArgs& a) {
   }
 }
 
-extern "C" __global__ __launch_bounds__(256) void rtq_act_prep_q8_0(ActArgs a) { act_prep<false>(a); }
-extern "C" __global__ __launch_bounds__(256) void rtq_act_prep_q8_k(ActArgs a) { act_prep<true>(a); }
+extern "C" __global__ __launch_bounds__(256) void rtq_act_prep_q8_0(ActArgs a) { act_prep<false, false>(a); }
+extern "C" __global__ __launch_bounds__(256) void rtq_act_prep_q8_k(ActArgs a) { act_prep<true, false>(a); }
+extern "C" __global__ __launch_bounds__(256) void rtq_act_prepn_q8_0(ActArgs a) { act_prep<false, true>(a); }
+extern "C" __global__ __launch_bounds__(256) void rtq_act_prepn_q8_k(ActArgs a) { act_prep<true, true>(a); }
 
 // The block-norm activation kernel on NT-token tiles (NT = 8 or 4): 16 / NT times act_prep's
 // workgroups for a given T, each reading NT rows whole for the sums of squares instead of 16.
@@ -725,15 +745,15 @@ template <int NT>
 __device__ __forceinline__ void act_prep_norm(const ActArgs& a) {
   static_assert(NT == 8 || NT == 4, "8- or 4-token tiles");
   constexpr int TPT = 256 / NT, RPW = NT / 4, BL = 32 / NT;  // threads per token, rows per wave, lanes per block
-  constexpr int KQ = RTQ_ACT_KQ, LDX = KQ + 1;
-  __shared__ float sx[16 * LDX];
-  __shared__ float sa[16 * LDX];
+  constexpr int KQ = RTQ_ACT_KQ;
+  __shared__ f4 sx[16 * KQ / 4];
+  __shared__ f4 sa[16 * KQ / 4];
   __shared__ float red[4 * 256];
   const int tid = threadIdx.x, tl = tid / TPT, sg = tid % TPT;
   const int t0 = blockIdx.x * NT, t = t0 + tl;
   const int Kc = a.Kp / 128;
   const int k0 = blockIdx.y * KQ, kk = k0 + sg * NT;
-  float mv[16];
+  f4 mv[4];
   if (a.A) lora_load_m(a.A, a.K, a.r, 0, k0, a.K, mv);  // uniform; in flight during the norm
   {
     // wave w normalises rows t0 + RPW w .. t0 + RPW w + RPW - 1 whole (as act_prep, every load issued first)
@@ -788,16 +808,19 @@ __device__ __forceinline__ void act_prep_norm(const ActArgs& a) {
           }
         }
       if (qy == 0 && lane == 0 && row < a.T) a.ninv[row] = ir;
-#pragma unroll
-      for (int e = 0; e < 4; e++) sx[(RPW * w + rr) * LDX + 4 * lane + e] = y[e];
+      sx[tile_unit(RPW * w + rr, lane)] = y;
     }
     // rows NT .. 15 of the LoRA product's token tile: zeros
-    for (int i = tid; i < (16 - NT) * LDX; i += 256) sx[NT * LDX + i] = 0.0f;
+    for (int i = tid; i < (16 - NT) * 64; i += 256) sx[NT * 64 + i] = f4{0.0f, 0.0f, 0.0f, 0.0f};
   }
   __syncthreads();
   float v[NT];
 #pragma unroll
-  for (int i = 0; i < NT; i++) v[i] = sx[tl * LDX + sg * NT + i];
+  for (int i = 0; i < NT / 4; i++) {
+    const f4 x4 = sx[tile_unit(tl, sg * (NT / 4) + i)];
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[4 * i + e] = x4[e];
+  }
   // Q8_0 codes: d = amax / 127 over the block (BL adjacent lanes), codes round(x / d)
   float amax = 0.0f;
 #pragma unroll
@@ -828,7 +851,7 @@ __device__ __forceinline__ void act_prep_norm(const ActArgs& a) {
       a.xdh[((int64_t)kc * a.Tp + t) * 4 + j] = real ? __builtin_bit_cast(uint16_t, (_Float16)dstore) : (uint16_t)0;
   }
   if (a.A)  // uniform
-    lora_partial_v<NT>(nullptr, mv, a.T, a.A, a.K, a.r, k0, a.K, t0, a.hp, gridDim.y, blockIdx.y, sx, sa, red);
+    lora_partial_v<NT>(mv, a.T, a.A, a.K, a.r, k0, a.K, t0, a.hp, gridDim.y, blockIdx.y, sx, sa, red);
 }
 extern "C" __global__ __launch_bounds__(256) void rtq_act_prep8_q8_0(ActArgs a) { act_prep_norm<8>(a); }
 extern "C" __global__ __launch_bounds__(256) void rtq_act_prep4_q8_0(ActArgs a) { act_prep_norm<4>(a); }
@@ -2689,10 +2712,9 @@ RTQ_GEMVQ(rtq_gemvq4_q6_k, FMT_Q6_K, RTQ_GQ_RG8, 4)
 //                         with gtok x >= T exit.
 // The dx kernel's extra workgroups sum the partials in slice order (h, and g scaled by s).
 extern "C" __global__ __launch_bounds__(256) void rtq_bwd_prep(BwdPrepArgs a) {
-  constexpr int KQ = RTQ_ACT_KQ, LDX = KQ + 1;
-  constexpr int SM = 16 * KQ + 64 > 16 * LDX ? 16 * KQ + 64 : 16 * LDX;  // A tile, or B slice (padded rows)
-  __shared__ float sx[16 * LDX];
-  __shared__ float sm[SM];
+  constexpr int KQ = RTQ_ACT_KQ;
+  __shared__ f4 sx[16 * KQ / 4];
+  __shared__ f4 sm[(16 * KQ + 64) / 4];  // A tile, or B slice (padded rows)
   __shared__ float red[4 * 256];
   const int y = (int)blockIdx.y + a.y0;
   if (y < a.nhq) {
@@ -2701,11 +2723,11 @@ extern "C" __global__ __launch_bounds__(256) void rtq_bwd_prep(BwdPrepArgs a) {
     const int t0 = blockIdx.x * a.gtok;
     if (t0 >= a.T) return;  // whole workgroup
     if (a.gtok == 64)
-      lora_up_partial<64>(a, t0, y - a.nhq, sm, red);
+      lora_up_partial<64>(a, t0, y - a.nhq, reinterpret_cast<float*>(sm), red);
     else if (a.gtok == 32)
-      lora_up_partial<32>(a, t0, y - a.nhq, sm, red);
+      lora_up_partial<32>(a, t0, y - a.nhq, reinterpret_cast<float*>(sm), red);
     else
-      lora_up_partial<16>(a, t0, y - a.nhq, sm, red);
+      lora_up_partial<16>(a, t0, y - a.nhq, reinterpret_cast<float*>(sm), red);
   }
 }
 

@@ -113,6 +113,8 @@ enum Kid {
   K_FILL,
   K_ACT_PREP,    // Q8_0 activations (Q4_0, Q8_0 weights)
   K_ACT_PREP_K,  // Q8_K activations (Q4_K, Q6_K weights)
+  K_ACT_PREPN,   // the same two of a block norm's input
+  K_ACT_PREPN_K,
   K_FWD_W,       // + format: wide forward GEMM
   K_FWD_S = K_FWD_W + F_COUNT,            // skinny (t <= 16)
   K_FWD_W_ISUMS = K_FWD_S + F_COUNT,      // debug variants writing the integer sums
@@ -168,7 +170,7 @@ enum Kid {
   K_COUNT = K_MODEL + KM_COUNT
 };
 constexpr const char* kKernelNames[] = {
-    "rtq_fill_zero",        "rtq_act_prep_q8_0",    "rtq_act_prep_q8_k",
+    "rtq_fill_zero",        "rtq_act_prep_q8_0",    "rtq_act_prep_q8_k",    "rtq_act_prepn_q8_0",   "rtq_act_prepn_q8_k",
     "rtq_fwd_q4_0_w",       "rtq_fwd_q8_0_w",       "rtq_fwd_q4_k_w",       "rtq_fwd_q6_k_w",
     "rtq_fwd_q4_0_s",       "rtq_fwd_q8_0_s",       "rtq_fwd_q4_k_s",       "rtq_fwd_q6_k_s",
     "rtq_fwd_q4_0_w_isums", "rtq_fwd_q8_0_w_isums", "rtq_fwd_q4_k_w_isums", "rtq_fwd_q6_k_w_isums",
@@ -746,7 +748,7 @@ rtq_status enqueue_forward(rtq_ctx* c, const rtq_weight* w, const float* x, int6
     ActArgs aa{x, (int)t, (int)w->cols, (int)p.Tp, (int)w->Kp, xq, xd, xg, gbias, lora ? la : nullptr, (int)r, hp,
                gp.gy > 1 ? y : nullptr, (int)w->rows, nullptr};
     act_in(aa);
-    RTQ_TRY(launch(c, is_kquant(w->type) ? K_ACT_PREP_K : K_ACT_PREP, dim3((unsigned)(p.Tp / 16), (unsigned)p.nhp),
+    RTQ_TRY(launch(c, (nf ? K_ACT_PREPN : K_ACT_PREP) + (is_kquant(w->type) ? 1 : 0), dim3((unsigned)(p.Tp / 16), (unsigned)p.nhp),
                    dim3(256), st, aa));
     FwdArgs fa{};
     fa.wq = w->wq;
@@ -852,7 +854,7 @@ rtq_status enqueue_forward(rtq_ctx* c, const rtq_weight* w, const float* x, int6
   // the block norms' activations (Q8_0 f16 fragments) on 8-token tiles: twice the workgroups, each
   // reading half the rows whole for the sums of squares (the same bits as the 16-token kernel)
   const int att = c->act_tt < 16 && nf && !kq && !mmi8 && !aa.zero_y && !aa.sg && !aa.xg ? c->act_tt : 16;
-  RTQ_TRY(launch(c, att == 8 ? K_ACT_PREP8 : att == 4 ? K_ACT_PREP4 : kq ? K_ACT_PREP_K : K_ACT_PREP,
+  RTQ_TRY(launch(c, att == 8 ? K_ACT_PREP8 : att == 4 ? K_ACT_PREP4 : (nf ? K_ACT_PREPN : K_ACT_PREP) + (kq ? 1 : 0),
                  dim3((unsigned)(p.Tp / att), (unsigned)p.nhp), dim3(256), st, aa));
   FwdArgs fa{};
   fa.wq = w->wq;
