@@ -84,6 +84,9 @@ struct ActArgs {
   // 1: the codes go to xq as int8 fragments of rtq_mmi8_* ([Tp/32][Kc][4][64] x 16 bytes, lane l:
   // token l % 32, the block's codes of k-groups 2 (l / 32) and 2 (l / 32) + 1), not f16 ones
   int xq_i8;
+  // Q8_K for rtq_mmk*_q4_k: 1: xd holds, instead of the replicated scales, the sums of 16 codes as f16
+  // [Kp/256][Tp][16], and xdh the super-blocks' d as f32 [Kp/256][Tp] (the two arrays' sizes)
+  int xbs;
   // or null: the activation is RMSNorm of na (+ nb) (src/ops.rs:14-35) with weight nw (+ noff), in
   // the order of rtq_m_rmsnorm's one-wave rows (K % 256 == 0, K <= 1024), formed here; the rows go
   // to x (then an output), na + nb to nh (with nb), 1 / rms to ninv (rows [T])
@@ -163,7 +166,7 @@ struct FwdArgs {
   float s;              // alpha / r
   int32_t* isums;       // debug: [T][N][K/32] (Q4_0, Q8_0), [T][N][K/256][2] (Q4_K: S1, S2),
                         // [T][N][K/256] (Q6_K: S), or null
-  const uint16_t* xdh;  // fp16 activation scales, layout of xd (rtq_mm_*)
+  const uint16_t* xdh;  // fp16 activation scales, layout of xd (rtq_mm_*); rtq_mmk*_q4_k: as ActArgs::xbs
   RankBlocks rb;        // LoRA B's block structure: a row's up-projection reads its member's ranks only
 };
 

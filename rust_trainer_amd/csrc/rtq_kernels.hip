@@ -707,8 +707,17 @@ __device__ __forceinline__ void act_prep(const ActArgs& a) {
       }
       }
       const bool real = t < a.T && kk < a.K;
-      if (hf == 0) a.xd[((int64_t)kc * a.Tp + t) * 4 + j] = real ? dstore : 0.0f;
-      if (a.xdh && hf == 0)  // Q8_0: dstore is an fp16 value
+      if (QK && a.xbs) {  // uniform: the super-block's d and the sums of 16 codes (rtq_mmk*_q4_k)
+        const int64_t o = (int64_t)blockIdx.y * a.Tp + t;
+        float s16 = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 16; i++) s16 += (float)q[i];
+        reinterpret_cast<_Float16*>(a.xd)[o * 16 + sg] = real ? (_Float16)s16 : (_Float16)0.0f;
+        if (sg == 0) reinterpret_cast<float*>(a.xdh)[o] = real ? dstore : 0.0f;
+      } else if (hf == 0) {
+        a.xd[((int64_t)kc * a.Tp + t) * 4 + j] = real ? dstore : 0.0f;
+      }
+      if (!QK && a.xdh && hf == 0)  // Q8_0: dstore is an fp16 value
         a.xdh[((int64_t)kc * a.Tp + t) * 4 + j] = real ? __builtin_bit_cast(uint16_t, (_Float16)dstore) : (uint16_t)0;
       if (a.xg && hf == 0) {  // Tp == 16: t is the token within the tile
         a.xg[(int64_t)(b * 2) * 16 + t] = real ? dstore : 0.0f;
@@ -1602,35 +1611,44 @@ extern "C" __global__ __launch_bounds__(256) void rtq_mm32_q4_0(FwdArgs a) { mm_
 extern "C" __global__ __launch_bounds__(256) void rtq_mm32_q8_0(FwdArgs a) { mm_tile<FMT_Q8_0, 2, RTQ_MM32_RING>(a); }
 
 // ============================================================== forward GEMM, large grids (Q4_K / Q6_K)
-// rtq_mm_*'s ring kernel for the K-quants: 128 weight rows x 16 TTN tokens (TTN 4 or 2), four
-// waves, wave w owning row groups 2w, 2w+1 x all token tiles, the half-chunk operands - codes
+// rtq_mm_*'s ring kernel for the K-quants: 128 weight rows x 16 TTN tokens (TTN 4), four
+// waves of two row groups x all token tiles, the half-chunk operands - codes
 // (Q4_K in the Q4_0 layout, Q6_K in the Q8_0 layout), the sub-block scale words of the 128 rows,
 // the activation codes (Q8_K values as exact f16) - copied global -> LDS by buffer loads with an
-// LDS destination into a RING-stage ring.  Arithmetic as fwd_tile's K-quant path: the 6-bit scales
-// folded into the f16 weight fragments (Q4_K: sc u and m; Q6_K: sh q and sl q), two f16 MFMAs per
-// block accumulate the super-block's exact integer sums S1, S2 over its four half chunks, and the
-// f32 epilogue runs once per super-block: Q4_K y += (d d_x) S1 - (dmin d_x) S2, Q6_K
-// y += (d d_x) (16 S1 + S2).  The super-block scales (d, dmin) of the lane's rows and the tokens'
-// Q8_K d are loaded from global memory at the super-block's first half chunk and used at its last.
+// LDS destination into a three-stage ring.  Arithmetic as fwd_tile's K-quant path: the 6-bit scales
+// folded into the f16 weight fragments, f16 MFMAs accumulate the super-block's exact integer sums
+// S1, S2 over its four half chunks, and the f32 epilogue runs once per super-block: Q4_K
+// y += (d d_x) S1 - (dmin d_x) S2, Q6_K y += (d d_x) (16 S1 + S2).  Q6_K folds sh and sl (two MFMAs
+// per block); Q4_K folds sc, and S2 = sum of m over the codes is one MFMA per super-block of the mins
+// against the activation kernel's sums of 16 codes (exact f16 integers, at most 2032) instead of one
+// per block.  The super-block's scales travel with its last half chunk's stage: loaded into registers
+// they cost two full drains of the ring per super-block (their waits cover every load in flight).
+// Bound by VALU (unpacking) plus MFMA issue.  Both changes, Q4_K 9728 x 2560 and 6144 x 2560 and 2560 x 4096
+// at 6792 tokens: 809 -> 682 us on average.
 template <int FMT, int TTN>
 struct MmkStage {  // one half chunk in LDS, in 16-byte units
   static constexpr int XQ = 0;                                           // [tt TTN][j2 2][lane 64] codes
   static constexpr int WQ = TTN * 2 * 64;                                // [rg 8][lane 64] Q4_K 8 B, Q6_K 16 B
   static constexpr int WK = WQ + (FMT == FMT_Q4_K ? 8 * 64 / 2 : 8 * 64);  // [rg 8][row 16] sub-block scale words
-  static constexpr int SIZE = WK + 8 * 4;
+  // a super-block's last half chunk: its (d, dmin) [rg 8][row 16], the tokens' d [64], Q4_K's code sums [t][2]
+  static constexpr int WS = WK + 8 * 4;
+  static constexpr int XS = WS + 8 * 4;
+  static constexpr int XB = XS + 16;
+  static constexpr int SIZE = XB + (FMT == FMT_Q4_K ? 16 * TTN * 2 : 0);
   static constexpr int NX = 2 * TTN;
   static constexpr int NWQ = FMT == FMT_Q4_K ? 16 : 8;
+  static constexpr int NXB = FMT == FMT_Q4_K ? TTN / 2 : 0;  // loads of code sums
 };
 
 template <int FMT, int TTN, int RING>
 __device__ __forceinline__ void mmk_tile(const FwdArgs& a) {
-  static_assert(TTN == 4 || TTN == 2, "64- or 32-token tiles");
+  constexpr int NW = 4, RW = 8 / NW;  // waves, row groups per wave
   using St = MmkStage<FMT, TTN>;
   extern __shared__ u4v mm_lds[];
   const int lane = threadIdx.x & 63, li = lane & 15, g = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int Kc = a.Kp / 128, nhc = a.Kp / 64;
-  const int ngroups = a.Np / 16, ntt = a.Tp / 16;
+  const int ngroups = a.Np / 16, ntt = (a.T + 16 * TTN - 1) / (16 * TTN) * TTN;  // whole tiles, <= Tp / 16
   constexpr int MM_GR = 8;
   const int nrb = (ngroups + 7) / 8, ntb = ntt / TTN, ntiles = nrb * ntb;
   const int id = blockIdx.x, xcd = id & 7, per = ntiles >> 3, rem = ntiles & 7;
@@ -1653,18 +1671,17 @@ __device__ __forceinline__ void mmk_tile(const FwdArgs& a) {
   const __amdgpu_buffer_rsrc_t rs_x = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.xq), (short)0, nb_x, 0x00020000);
   const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.wq), (short)0, nb_w, 0x00020000);
   const __amdgpu_buffer_rsrc_t rs_wd = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.wd), (short)0, nb_wd, 0x00020000);
-  constexpr int KX = St::NX / 4, KW = St::NWQ / 4;
-  static_assert(St::NX % 4 == 0 && St::NWQ % 4 == 0, "load split over four waves");
-  uint32_t vx[KX], vw[KW], ve = 0;
+  constexpr int KW = St::NWQ / NW, KX = St::NX / NW;
+  static_assert(St::NWQ % NW == 0 && St::NX % NW == 0 && St::NXB <= 2, "load split over the waves");
+  uint32_t vx[KX], vw[KW], ve = 0, vs = 0;
 #pragma unroll
   for (int k = 0; k < KX; k++) {
-    const int i = w + 4 * k;
-    const uint32_t ttg = (uint32_t)min(tt0 + (i >> 1), ntt - 1);
-    vx[k] = ((ttg * Kc * 4 + (i & 1)) * 64 + lane) * 16;
+    const int i = w + NW * k;
+    vx[k] = (((uint32_t)(tt0 + (i >> 1)) * Kc * 4 + (i & 1)) * 64 + lane) * 16;
   }
 #pragma unroll
   for (int k = 0; k < KW; k++) {
-    const int iw = w + 4 * k;
+    const int iw = w + NW * k;
     if (FMT == FMT_Q4_K) {
       const int wi = (iw & 1) * 64 + lane;
       const uint32_t rgg = (uint32_t)min(rg0 + (iw >> 1), ngroups - 1);
@@ -1679,15 +1696,31 @@ __device__ __forceinline__ void mmk_tile(const FwdArgs& a) {
     const uint32_t rgg = (uint32_t)min(rg0 + (wi >> 4), ngroups - 1);
     ve = ((rgg * Kc * 16 + (wi & 15)) * 2) * 4;
   }
+  // a super-block's scales, one load each by waves NW - 1 (tokens' d), NW - 2 and NW - 3 (d, dmin of rows
+  // 64 i ..), and 0 .. NXB - 1 (code sums of tokens 32 i ..)
+  const int sk = w == NW - 1 ? 0 : w >= NW - 3 ? 1 : -1;  // kind of this wave's load among the first two
+  if (sk == 0) {
+    const uint32_t t = (uint32_t)min(tt0 * 16 + lane, a.Tp - 1);
+    vs = FMT == FMT_Q4_K ? t * 4 : t * 16;
+  } else if (sk == 1) {
+    const int wi = (NW - 2 - w) * 64 + lane;
+    vs = ((uint32_t)min(rg0 + (wi >> 4), ngroups - 1) * (Kc >> 1) * 16 + (wi & 15)) * 4;
+  }
+  const uint32_t vb = ((uint32_t)(tt0 * 16 + 32 * w) * 2 + lane) * 16;  // code sums: two 16-byte units a token
+  const uint32_t nb_d = (uint32_t)(Kc >> 1) * a.Tp * (FMT == FMT_Q4_K ? 4 : 32), nb_ws = (uint32_t)ngroups * (Kc >> 1) * 64;
+  const __amdgpu_buffer_rsrc_t rs_d = make_rsrc(FMT == FMT_Q4_K ? (const void*)a.xdh : (const void*)a.xd, nb_d);
+  const __amdgpu_buffer_rsrc_t rs_ws = make_rsrc(a.wsb, nb_ws);
+  const __amdgpu_buffer_rsrc_t rs_b = make_rsrc(a.xd, (uint32_t)(Kc >> 1) * a.Tp * 32);
+  const int nsl = (sk >= 0 ? 1 : 0) + (w < St::NXB ? 1 : 0);  // this wave's loads of a super-block's scales
   auto issue = [&](int st, int hc) {
     u4v* S = mm_lds + st * St::SIZE;
     const uint32_t kc = hc >> 1, h = hc & 1;
 #pragma unroll
     for (int k = 0; k < KX; k++)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_x, RTQ_LDSP(S + St::XQ + (w + 4 * k) * 64), 16, vx[k], hc * 2048u, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_x, RTQ_LDSP(S + St::XQ + (w + NW * k) * 64), 16, vx[k], hc * 2048u, 0, 0);
 #pragma unroll
     for (int k = 0; k < KW; k++) {
-      const int iw = w + 4 * k;
+      const int iw = w + NW * k;
       if (FMT == FMT_Q4_K)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_w, RTQ_LDSP(S + St::WQ + (iw >> 1) * 32 + (iw & 1) * 16), 4, vw[k],
                                                  kc * 1024u + h * 8u, 0, 0);
@@ -1696,43 +1729,59 @@ __device__ __forceinline__ void mmk_tile(const FwdArgs& a) {
     }
     if (w < 2)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_wd, RTQ_LDSP(S + St::WK + w * 16), 4, ve, kc * 128u + h * 4u, 0, 0);
+    if ((hc & 3) == 3) {
+      const uint32_t sb = hc >> 2;
+      if (sk == 0)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_d, RTQ_LDSP(S + St::XS), 4, vs, sb * a.Tp * (FMT == FMT_Q4_K ? 4u : 32u), 0, 0);
+      else if (sk == 1)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_ws, RTQ_LDSP(S + St::WS + (NW - 2 - w) * 16), 4, vs, sb * 64u, 0, 0);
+      if (w < St::NXB)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_b, RTQ_LDSP(S + St::XB + w * 64), 16, vb, sb * a.Tp * 32u, 0, 0);
+    }
   };
 
   const f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-  f4 acc[TTN][2], s1[TTN][2], s2[TTN][2];
+  f4 acc[TTN][RW], s1[TTN][RW], s2[TTN][RW];
 #pragma unroll
   for (int i = 0; i < TTN; i++)
 #pragma unroll
-    for (int r = 0; r < 2; r++) acc[i][r] = s1[i][r] = s2[i][r] = zero;
-  u4v esb[2];     // (d | dmin << 16) of rows 4g .. 4g + 3 of row groups 2w, 2w + 1, this super-block
-  float xsb[TTN]; // the tokens' Q8_K d of this super-block (token li of each tile)
+    for (int r = 0; r < RW; r++) acc[i][r] = s1[i][r] = s2[i][r] = zero;
+  u4v mf[RW];  // Q4_K: row li's mins of half blocks 8g .. 8g + 7 of the super-block (g < 2; zeros else), f16 pairs
+#pragma unroll
+  for (int r = 0; r < RW; r++) mf[r] = u4v{0u, 0u, 0u, 0u};
   auto compute = [&](int st, int hc) {
     const u4v* S = mm_lds + st * St::SIZE;
-    if ((hc & 3) == 0) {  // a super-block starts: its scales, consumed at its last half chunk
-      const int sb = hc >> 2;
+    uint32_t kw[RW];
 #pragma unroll
-      for (int r = 0; r < 2; r++)
-        esb[r] = reinterpret_cast<const u4v*>(a.wsb)[((uint32_t)min(rg0 + 2 * w + r, ngroups - 1) * (Kc >> 1) + sb) * 4 + g];
+    for (int r = 0; r < RW; r++) kw[r] = reinterpret_cast<const uint32_t*>(S + St::WK)[(RW * w + r) * 16 + li];
+    if (FMT == FMT_Q4_K) {  // mins of blocks 2 (hc & 3), + 1: half blocks 4 (hc & 1) .. + 3 of lane group (hc & 3) / 2
+      const bool mine = g == ((hc >> 1) & 1);
 #pragma unroll
-      for (int i = 0; i < TTN; i++)
-        xsb[i] = a.xd[((int64_t)(2 * sb) * a.Tp + min((tt0 + i) * 16 + li, a.Tp - 1)) * 4];
+      for (int r = 0; r < RW; r++) {
+        const uint32_t m2 = (kw[r] >> 8) & 0x003f003fu;  // block 2h low, 2h + 1 high
+        const uint32_t mw = __builtin_bit_cast(uint32_t, sub_h2(m2 | 0x64006400u, (_Float16)1024.0f));
+        const uint32_t lo = __builtin_amdgcn_perm(mw, mw, 0x01000100u), hi = __builtin_amdgcn_perm(mw, mw, 0x03020302u);
+        if (hc & 1) {
+          mf[r].z = mine ? lo : mf[r].z;
+          mf[r].w = mine ? hi : mf[r].w;
+        } else {
+          mf[r].x = mine ? lo : mf[r].x;
+          mf[r].y = mine ? hi : mf[r].y;
+        }
+      }
     }
 #pragma unroll
     for (int j2 = 0; j2 < 2; j2++) {
-      half8 f1[2], f2[2];
+      half8 f1[RW], f2[RW];
 #pragma unroll
-      for (int r = 0; r < 2; r++) {
-        const int rl = 2 * w + r;
-        const uint32_t kw = reinterpret_cast<const uint32_t*>(S + St::WK)[rl * 16 + li];
-        const uint32_t wv = j2 ? (kw >> 16) : kw;
+      for (int r = 0; r < RW; r++) {
+        const uint32_t wv = j2 ? (kw[r] >> 16) : kw[r];
         if (FMT == FMT_Q4_K) {
-          const u2v q2 = reinterpret_cast<const u2v*>(S + St::WQ)[rl * 64 + lane];
-          const _Float16 sc = (_Float16)(float)(wv & 0x3fu), m = (_Float16)(float)((wv >> 8) & 0x3fu);
+          const u2v q2 = reinterpret_cast<const u2v*>(S + St::WQ)[(RW * w + r) * 64 + lane];
+          const _Float16 sc = (_Float16)(float)(wv & 0x3fu);
           f1[r] = q4_0_frag<0>(j2 ? q2.y : q2.x) * sc;
-          const half8 mm = {m, m, m, m, m, m, m, m};
-          f2[r] = mm;
         } else {
-          const u4v qv = S[St::WQ + rl * 64 + lane];
+          const u4v qv = S[St::WQ + (RW * w + r) * 64 + lane];
           const int s0 = (int)(int8_t)(wv & 0xffu), s1v = (int)(int8_t)((wv >> 8) & 0xffu);
           const _Float16 h0 = (_Float16)(float)(s0 >> 4), h1 = (_Float16)(float)(s1v >> 4);
           const _Float16 l0 = (_Float16)(float)(s0 & 15), l1 = (_Float16)(float)(s1v & 15);
@@ -1746,23 +1795,32 @@ __device__ __forceinline__ void mmk_tile(const FwdArgs& a) {
       for (int i = 0; i < TTN; i++) {
         const half8 xf = __builtin_bit_cast(half8, S[St::XQ + (i * 2 + j2) * 64 + lane]);
 #pragma unroll
-        for (int r = 0; r < 2; r++) {
+        for (int r = 0; r < RW; r++) {
           s1[i][r] = mfma_f16(f1[r], xf, s1[i][r]);
-          s2[i][r] = mfma_f16(f2[r], xf, s2[i][r]);
+          if (FMT == FMT_Q6_K) s2[i][r] = mfma_f16(f2[r], xf, s2[i][r]);
         }
       }
     }
     if ((hc & 3) == 3) {  // the super-block's f32 epilogue, then the sums restart
+      u4v esb[RW];        // (d | dmin << 16) of rows 4g .. 4g + 3 of the row group
 #pragma unroll
-      for (int i = 0; i < TTN; i++)
+      for (int r = 0; r < RW; r++) esb[r] = S[St::WS + (RW * w + r) * 4 + g];
 #pragma unroll
-        for (int r = 0; r < 2; r++) {
+      for (int i = 0; i < TTN; i++) {
+        const float xsb = reinterpret_cast<const float*>(S + St::XS)[i * 16 + li];
+        if (FMT == FMT_Q4_K) {  // lane groups 2, 3: zero mins against sums of 0, 1
+          const half8 xb = __builtin_bit_cast(half8, S[St::XB + (i * 16 + li) * 2 + (g & 1)]);
+#pragma unroll
+          for (int r = 0; r < RW; r++) s2[i][r] = mfma_f16(__builtin_bit_cast(half8, mf[r]), xb, zero);
+        }
+#pragma unroll
+        for (int r = 0; r < RW; r++) {
 #pragma unroll
           for (int e = 0; e < 4; e++) {
             const uint32_t ev = comp(esb[r], e);
-            const float dd = h2f((uint16_t)(ev & 0xffffu)) * xsb[i];
+            const float dd = h2f((uint16_t)(ev & 0xffffu)) * xsb;
             if (FMT == FMT_Q4_K) {
-              const float dm = h2f((uint16_t)(ev >> 16)) * xsb[i];
+              const float dm = h2f((uint16_t)(ev >> 16)) * xsb;
               acc[i][r][e] = fmaf(dd, s1[i][r][e], fmaf(-dm, s2[i][r][e], acc[i][r][e]));
             } else {
               acc[i][r][e] = fmaf(dd, fmaf(16.0f, s1[i][r][e], s2[i][r][e]), acc[i][r][e]);
@@ -1771,11 +1829,13 @@ __device__ __forceinline__ void mmk_tile(const FwdArgs& a) {
           s1[i][r] = zero;
           s2[i][r] = zero;
         }
+      }
     }
   };
 
-  static_assert(RING >= 3 && (RING - 2) * (KX + KW + 1) <= 63, "ring depth within the load counter");
-  constexpr int MINL = KX + KW;
+  // every wave's loads per stage, at least; a stage that ends a super-block adds nsl
+  constexpr int MINL = KW + KX;
+  static_assert(RING == 3 && MINL + 2 <= 63, "one stage in flight behind the one waited for");
 #pragma unroll
   for (int s = 0; s < RING - 1; s++)
     if (s < nhc) issue(s, s);
@@ -1784,7 +1844,14 @@ __device__ __forceinline__ void mmk_tile(const FwdArgs& a) {
     for (int u = 0; u < RING; u++) {
       const int hc = hc0 + u;
       if (hc < nhc) {
-        vm_wait_stages<MINL>(min(RING - 2, nhc - 1 - hc));
+        if (hc + 1 == nhc)
+          __builtin_amdgcn_s_waitcnt(vm_wait_imm(0));
+        else if (((hc + 1) & 3) == 3 && nsl == 1)
+          __builtin_amdgcn_s_waitcnt(vm_wait_imm(MINL + 1));
+        else if (((hc + 1) & 3) == 3 && nsl == 2)
+          __builtin_amdgcn_s_waitcnt(vm_wait_imm(MINL + 2));
+        else
+          __builtin_amdgcn_s_waitcnt(vm_wait_imm(MINL));
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         if (hc + RING - 1 < nhc) issue((u + RING - 1) % RING, hc + RING - 1);
@@ -1798,41 +1865,42 @@ __device__ __forceinline__ void mmk_tile(const FwdArgs& a) {
   float(*sh)[RTQ_LDS_RANK + 1] = reinterpret_cast<float(*)[RTQ_LDS_RANK + 1]>(mm_lds);
   float(*sbm)[RTQ_LDS_RANK + 1] = sh + 16 * TTN;
   int span0 = 0, span1 = 0;
-  int win0[2] = {0, 0}, win1[2] = {0, 0};
+  int win0[RW] = {}, win1[RW] = {};
   if (lora) {
     rb_span(a.rb, a.r, rg0 * 16, min(rg0 * 16 + 128, a.N), span0, span1);
 #pragma unroll
-    for (int r = 0; r < 2; r++) rb_span(a.rb, a.r, (rg0 + 2 * w + r) * 16, (rg0 + 2 * w + r) * 16 + 16, win0[r], win1[r]);
+    for (int r = 0; r < RW; r++) rb_span(a.rb, a.r, (rg0 + RW * w + r) * 16, (rg0 + RW * w + r) * 16 + 16, win0[r], win1[r]);
   }
-  f4 lacc[TTN][2];
+  f4 lacc[TTN][RW];
 #pragma unroll
   for (int i = 0; i < TTN; i++)
 #pragma unroll
-    for (int r = 0; r < 2; r++) lacc[i][r] = zero;
+    for (int r = 0; r < RW; r++) lacc[i][r] = zero;
   for (int c0 = span0; c0 < span1; c0 += RTQ_LDS_RANK) {
     const int c1 = min(c0 + RTQ_LDS_RANK, span1);
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     for (int j0 = c0; j0 < c1; j0 += 16) {
-      float hv[8], bv[8];
+      constexpr int PE = 128 * 16 / (64 * NW);
+      float hv[PE], bv[PE];
 #pragma unroll
-      for (int k = 0; k < 8; k++) {
-        const int e = threadIdx.x + 256 * k, tl = e >> 4, j = min(j0 + (e & 15), a.r - 1);
+      for (int k = 0; k < PE; k++) {
+        const int e = threadIdx.x + 64 * NW * k, tl = e >> 4, j = min(j0 + (e & 15), a.r - 1);
         hv[k] = tl < 16 * TTN ? sum_partials(a.hp, (int64_t)min(tt0 * 16 + tl, a.T - 1) * a.r + j, a.nhp) : 0.0f;
         bv[k] = a.lb[(int64_t)min(rg0 * 16 + tl, a.N - 1) * a.r + j];
       }
 #pragma unroll
-      for (int k = 0; k < 8; k++) {
-        const int e = threadIdx.x + 256 * k, jl = j0 - c0 + (e & 15);
+      for (int k = 0; k < PE; k++) {
+        const int e = threadIdx.x + 64 * NW * k, jl = j0 - c0 + (e & 15);
         if ((e >> 4) < 16 * TTN) sh[e >> 4][jl] = hv[k];
         sbm[e >> 4][jl] = bv[k];
       }
     }
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < 2; r++) {
+    for (int r = 0; r < RW; r++) {
       const int lo = max(win0[r], c0), hi = min(win1[r], c1);
-      const int nb0 = (rg0 + 2 * w + r) * 16, rl = (2 * w + r) * 16;
+      const int nb0 = (rg0 + RW * w + r) * 16, rl = (RW * w + r) * 16;
       for (int j0 = lo; j0 < hi; j0 += 4) {
         const int j = j0 + g, jl = min(j, hi - 1) - c0;
         const float bv = (nb0 + li < a.N && j < hi) ? sbm[rl + li][jl] : 0.0f;
@@ -1847,9 +1915,9 @@ __device__ __forceinline__ void mmk_tile(const FwdArgs& a) {
 #pragma unroll
   for (int i = 0; i < TTN; i++) {
 #pragma unroll
-    for (int r = 0; r < 2; r++) {
+    for (int r = 0; r < RW; r++) {
       const int t = tt0 * 16 + i * 16 + li;
-      const int nb0 = (rg0 + 2 * w + r) * 16, n0 = nb0 + 4 * g;
+      const int nb0 = (rg0 + RW * w + r) * 16, n0 = nb0 + 4 * g;
       if (nb0 >= a.N) continue;
       if (t < a.T) {
         f4 v = acc[i][r];
@@ -1875,8 +1943,6 @@ __device__ __forceinline__ void mmk_tile(const FwdArgs& a) {
 
 extern "C" __global__ __launch_bounds__(256) void rtq_mmk64_q4_k(FwdArgs a) { mmk_tile<FMT_Q4_K, 4, RTQ_MM64_RING>(a); }
 extern "C" __global__ __launch_bounds__(256) void rtq_mmk64_q6_k(FwdArgs a) { mmk_tile<FMT_Q6_K, 4, RTQ_MM64_RING>(a); }
-extern "C" __global__ __launch_bounds__(256) void rtq_mmk32_q4_k(FwdArgs a) { mmk_tile<FMT_Q4_K, 2, RTQ_MM32_RING>(a); }
-extern "C" __global__ __launch_bounds__(256) void rtq_mmk32_q6_k(FwdArgs a) { mmk_tile<FMT_Q6_K, 2, RTQ_MM32_RING>(a); }
 
 // ============================================================== forward GEMM on int8 MFMA (Q4_0 / Q8_0)
 // rtq_mm64_*'s tiles (128 weight rows x 16 TTN tokens, TTN 4 here, four waves, the same RING-stage

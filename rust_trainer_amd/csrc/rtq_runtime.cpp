@@ -136,10 +136,8 @@ enum Kid {
   K_MM32_Q8_0,
   K_MMI8_64_Q4_0,  // the 128 x 64 tiles with the block sums on int8 MFMA
   K_MMI8_64_Q8_0,
-  K_MMK64_Q4_K,    // the LDS-ring kernel for the K-quants: 128 x 64 and 128 x 32 tiles
+  K_MMK64_Q4_K,    // the LDS-ring kernel for the K-quants: 128 x 64 tiles
   K_MMK64_Q6_K,
-  K_MMK32_Q4_K,
-  K_MMK32_Q6_K,
   K_BWD_PREP,
   K_DX,          // + format
   K_DX16 = K_DX + F_COUNT,  // + format: t <= 16
@@ -183,7 +181,7 @@ constexpr const char* kKernelNames[] = {
     "rtq_mm_q4_0",          "rtq_mm_q8_0",
     "rtq_mm64_q4_0",        "rtq_mm64_q8_0",        "rtq_mm32_q4_0",        "rtq_mm32_q8_0",
     "rtq_mmi8_64_q4_0",     "rtq_mmi8_64_q8_0",
-    "rtq_mmk64_q4_k",       "rtq_mmk64_q6_k",       "rtq_mmk32_q4_k",       "rtq_mmk32_q6_k",
+    "rtq_mmk64_q4_k",       "rtq_mmk64_q6_k",
     "rtq_bwd_prep",
     "rtq_dx_q4_0",          "rtq_dx_q8_0",          "rtq_dx_q4_k",          "rtq_dx_q6_k",
     "rtq_dx16_q4_0",        "rtq_dx16_q8_0",        "rtq_dx16_q4_k",        "rtq_dx16_q6_k",
@@ -242,8 +240,8 @@ struct rtq_ctx {
   int g64_min = -1;   // fewest 64-token g-partial workgroups (else 16-token ones): -1 = CUs / 2 (RTQ_G64_MIN)
   int fwd_mm = -1;    // large-grid forward: -1 automatic, 0 never, 1 / 2 / 3 the 128- / 64- / 32-token tiles
                       // whenever the format allows (RTQ_FWD_MM)
-  int fwd_mmk = -1;   // K-quant ring forward (rtq_mmk*_*; RTQ_FWD_MMK): -1 automatic, 0 never, 1 / 2 the 64- /
-                      // 32-token tiles whenever the shape allows
+  int fwd_mmk = -1;   // K-quant ring forward (rtq_mmk64_*; RTQ_FWD_MMK): -1 automatic, 0 never, else whenever
+                      // the shape allows
   int dxv = 1;        // t == 1 dx on f32 FMAs (rtq_dxv1_*; RTQ_DXV=0: rtq_dx16_*)
   int dxv_wpc = 3;    // rtq_dxv1_* row splits for about this many workgroups per CU (RTQ_DXV_WPC)
   int gemvq = 1;      // one-launch GEMV for t <= 4 (rtq_gemvq*_*; RTQ_GEMVQ=0: activation kernel + GEMM)
@@ -404,7 +402,8 @@ unsigned mm_lds_bytes(int type, int ttn, int ring) {  // ttn: token tiles of 16 
 }
 // rtq_mmk*_* (K-quants, ttn 4 or 2): codes, sub-block scale words and activation codes per stage
 unsigned mmk_lds_bytes(int type, int ttn, int ring) {
-  const unsigned stage = 16u * (ttn * 2 * 64 + (type == RTQ_TYPE_Q4_K ? 8 * 64 / 2 : 8 * 64) + 8 * 4);
+  const unsigned stage = 16u * (ttn * 2 * 64 + (type == RTQ_TYPE_Q4_K ? 8 * 64 / 2 : 8 * 64) + 8 * 4 +
+                                8 * 4 + 16 + (type == RTQ_TYPE_Q4_K ? 16 * ttn * 2 : 0));  // super-block scales, code sums
   return std::max((unsigned)ring * stage, (16u * ttn + 128u) * (RTQ_LDS_RANK + 1) * 4u);
 }
 // rtq_mmi8_* (ttn 4): int8 activation fragments, half the f16 ones' bytes
@@ -818,16 +817,13 @@ rtq_status enqueue_forward(rtq_ctx* c, const rtq_weight* w, const float* x, int6
   const bool mmi8 = mm && (mm_ttn == 8 || mm_ttn == 4) &&
                     (c->fwd_i8 == 1 || (c->fwd_i8 < 0 && w->type == RTQ_TYPE_Q8_0));
   if (mmi8) mm_ttn = 4;
-  // K-quants: the LDS-ring kernel on 64-token tiles where they give every CU a workgroup, else on
-  // 32-token tiles where those do.  Measured per forward call at 2048 tokens against the tile
-  // kernel (rtq_fwd_*_w): Qwen3-4B q | k | v 226 -> 179 us, gate | up 641 -> 464, down (Q6_K) 384
-  // -> 323, LM head Q4_K 1778 -> 1307 (32-token tiles: 214, 585, 375, 1673)
-  int mmk_ttn = 0;
-  if (!p.skinny && !isums && is_kquant(w->type)) {
-    if (c->fwd_mmk == 1) mmk_ttn = 4;
-    else if (c->fwd_mmk == 2) mmk_ttn = 2;
-    else if (c->fwd_mmk < 0) mmk_ttn = mm64 >= c->cu_count ? 4 : (mm32 >= c->cu_count ? 2 : 0);
-  }
+  // K-quants: the LDS-ring kernel where its 128 x 64 tiles (of tokens < t) give half the CUs two workgroups,
+  // else the tile kernel (rtq_fwd_*_w).  Measured per forward kernel, ring / tile, us (and workgroups):
+  // Q4_K 9728 x 2560 at 200, 400, 1001 tokens 49 / 42 (304), 64 / 70 (532), 108 / 147 (1216); Q6_K 2560 x
+  // 9728 at 1001, 2048 183 / 143 (320), 291 / 306 (640); Q4_K 2560 x 4096 at 1001, 2048 74 / 61 (320),
+  // 101 / 115 (640); Q4_K 14336 x 4096 at 100, 200 58 / 48 (224), 77 / 81 (448)
+  const int64_t mmk_tiles = mm_rows * cdiv(t, 64);
+  const bool mmk = !p.skinny && !isums && kq && (c->fwd_mmk > 0 || (c->fwd_mmk < 0 && 2 * mmk_tiles >= 3 * c->cu_count));
   const int64_t mm_tiles = mm_ttn == 8 ? mm128 : mm_ttn == 4 ? mm64 : mm32;
   // split K across workgroups when the output alone gives too few of them (atomics into a
   // zeroed y); every split keeps at least one half chunk per wave (K-quants: one super-block of
@@ -837,7 +833,7 @@ rtq_status enqueue_forward(rtq_ctx* c, const rtq_weight* w, const float* x, int6
   // get the same bits
   const int64_t tiles = gx * gy;
   int64_t ks = 1;
-  if (!isums && !mm && !mmk_ttn && !w8 && tiles < c->cu_count) {
+  if (!isums && !mm && !mmk && !w8 && tiles < c->cu_count) {
     const int64_t want = cdiv(p.skinny ? 2 * c->cu_count : c->cu_count, tiles);
     ks = std::max<int64_t>(1, std::min<int64_t>(want, Kc / (kq ? 8 : 2)));
   }
@@ -845,12 +841,14 @@ rtq_status enqueue_forward(rtq_ctx* c, const rtq_weight* w, const float* x, int6
   if (kq) kcps = roundup(kcps, 2);
   ks = cdiv(Kc, kcps);
 
-  uint16_t* xdh = mm ? ar.take<uint16_t>(p.xdh_bytes / 2) : nullptr;
+  const bool xbs = mmk && w->type == RTQ_TYPE_Q4_K;  // code sums instead of the replicated scales
+  uint16_t* xdh = mm || xbs ? ar.take<uint16_t>(p.xdh_bytes / 2) : nullptr;
   if (ar.off > ar.cap) return fail(RTQ_ERR_INVALID, "internal: workspace too small");
   ActArgs aa{x, (int)t, (int)w->cols, (int)p.Tp, (int)w->Kp, xq, xd, nullptr, 0.0f, lora ? la : nullptr, (int)r, hp,
              ks > 1 ? y : nullptr, (int)w->rows, xdh};
   act_in(aa);
   aa.xq_i8 = mmi8 ? 1 : 0;
+  aa.xbs = xbs ? 1 : 0;
   // the block norms' activations (Q8_0 f16 fragments) on 8-token tiles: twice the workgroups, each
   // reading half the rows whole for the sums of squares (the same bits as the 16-token kernel)
   const int att = c->act_tt < 16 && nf && !kq && !mmi8 && !aa.zero_y && !aa.sg && !aa.xg ? c->act_tt : 16;
@@ -886,12 +884,11 @@ rtq_status enqueue_forward(rtq_ctx* c, const rtq_weight* w, const float* x, int6
   if (mmi8)
     return launch(c, K_MMI8_64_Q4_0 + (w->type == RTQ_TYPE_Q4_0 ? 0 : 1), dim3((unsigned)mm_tiles), dim3(256), st, fa,
                   mmi8_lds_bytes(w->type, 4, RTQ_MM64_RING));
-  if (mmk_ttn) {
-    if (!fa.wq || !fa.wd || !fa.wsb || !fa.xq || !fa.xd || !fa.y)
+  if (mmk) {
+    if (!fa.wq || !fa.wd || !fa.wsb || !fa.xq || !fa.xd || !fa.y || (xbs && !fa.xdh))
       return fail(RTQ_ERR_INVALID, "internal: rtq_mmk_* operand missing");
-    const int kid = (mmk_ttn == 4 ? K_MMK64_Q4_K : K_MMK32_Q4_K) + (w->type == RTQ_TYPE_Q4_K ? 0 : 1);
-    return launch(c, kid, dim3((unsigned)(mmk_ttn == 4 ? mm64 : mm32)), dim3(256), st, fa,
-                  mmk_lds_bytes(w->type, mmk_ttn, mmk_ttn == 4 ? RTQ_MM64_RING : RTQ_MM32_RING));
+    return launch(c, K_MMK64_Q4_K + (w->type == RTQ_TYPE_Q4_K ? 0 : 1), dim3((unsigned)mmk_tiles), dim3(256), st, fa,
+                  mmk_lds_bytes(w->type, 4, RTQ_MM64_RING));
   }
   if (mm) {
     const int ring = mm_ttn == 8 ? RTQ_MM_RING : mm_ttn == 4 ? RTQ_MM64_RING : RTQ_MM32_RING;

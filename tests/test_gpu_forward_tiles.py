@@ -1,0 +1,56 @@
+"""The large-grid forward kernels at the edges of their token tiles, each forced by its knob, against the
+oracle: token counts that leave the last 32-, 64- or 128-token tile nearly empty or full (tiles of tokens
+past the last are not launched), ragged rows, one super-block and several.  Rows of equal activations put
+every code at 127, so the Q4_K kernel's sums of 16 codes are at their largest (2032), against weights whose
+minima are at theirs.  y is an f32 sum of K / 32 (K / 256) block terms; both sides round each once, so 2e-6
+of the largest value holds for the K here."""
+import os
+
+import numpy as np
+import pytest
+
+import oracle as O
+import rust_trainer_amd as rt
+
+pytestmark = pytest.mark.gpu
+
+KNOBS = {"mmk": {"RTQ_FWD_MMK": "1"}, "auto": {}}
+
+
+@pytest.fixture(scope="module", params=list(KNOBS))
+def ctx(request):
+    knobs = KNOBS[request.param]
+    old = {k: os.environ.get(k) for k in knobs}
+    os.environ.update(knobs)
+    try:
+        c = rt.Context(0)
+    finally:
+        for k, v in old.items():
+            if v is None:
+                del os.environ[k]
+            else:
+                os.environ[k] = v
+    c.formats = (O.Q4_K, O.Q6_K) if request.param == "mmk" else (O.Q4_0, O.Q8_0) if knobs else (O.Q4_0, O.Q8_0, O.Q4_K, O.Q6_K)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("n,k,t", [(130, 256, 17), (64, 512, 32), (200, 768, 33), (130, 512, 64), (257, 256, 65), (128, 512, 128),
+                                   (144, 256, 129)])
+def test_forward_token_tiles(ctx, n, k, t):
+    for wtype in ctx.formats:
+        w = O.Rng(1).vec_normal(n * k, 0.02).reshape(n, k)
+        w[: n // 2, : k // 2] = -0.05 + 0.001 * w[: n // 2, : k // 2]  # nearly all minimum
+        x = O.Rng(2).vec_normal(t * k, 1.0).reshape(t, k)
+        x[::3] = 0.75  # every code 127
+        a = O.Rng(3).vec_normal(5 * k, 0.05).reshape(5, k)
+        b = O.Rng(4).vec_normal(n * 5, 0.05).reshape(n, 5)
+        blocks = O.quantize(wtype, w)
+        lin = rt.Linear("tiles", rt.HipFrozen(wtype, blocks, n, k, ctx=ctx))
+        y = lin.forward(x, t).reshape(t, n)
+        want = np.asarray(O.frozen_forward(wtype, blocks, n, k, x, nthreads=8), np.float64).reshape(t, n)
+        assert np.abs(y - want).max() <= 2e-6 * np.abs(want).max(), wtype
+        lin.lora = rt.Lora(5, 10.0, a, b)
+        y = lin.forward(x, t).reshape(t, n)
+        want = want + 2 * (x.astype(np.float64) @ a.T.astype(np.float64)) @ b.T.astype(np.float64)
+        assert np.abs(y - want).max() <= 2e-6 * np.abs(want).max(), wtype
