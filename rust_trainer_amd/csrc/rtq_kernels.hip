@@ -1344,7 +1344,7 @@ __device__ __forceinline__ void mm_tile(const FwdArgs& a) {
   const int lane = threadIdx.x & 63, li = lane & 15, g = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int Kc = a.Kp / 128, nhc = a.Kp / 64;
-  const int ngroups = a.Np / 16, ntt = a.Tp / 16;
+  const int ngroups = a.Np / 16, ntt = (a.T + 16 * TTN - 1) / (16 * TTN) * TTN;  // whole tiles of tokens < T
   // XCD-aware tile order: workgroup id -> (XCD id % 8, slot id / 8) -> a contiguous range of the
   // tile order per XCD.  The order takes the row blocks in groups of MM_GR: within a group token
   // block by token block, the group's row blocks of one token block consecutive.  The ~64
@@ -1988,7 +1988,7 @@ __device__ __forceinline__ void mmi8_tile(const FwdArgs& a) {
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int Kc = a.Kp / 128, nhc = a.Kp / 64;
-  const int ngroups = a.Np / 16, ntt = a.Tp / 16, ntt32 = a.Tp / 32;
+  const int ngroups = a.Np / 16, ntt = (a.T + 16 * TTN - 1) / (16 * TTN) * TTN, ntt32 = a.Tp / 32;
   // tile order as rtq_mm_*: XCD-aware, row blocks in groups of MM_GR per token-block sweep
   constexpr int MM_GR = 8;
   const int nrb = (ngroups + 7) / 8, ntb = ntt / TTN, ntiles = nrb * ntb;

@@ -792,31 +792,39 @@ rtq_status enqueue_forward(rtq_ctx* c, const rtq_weight* w, const float* x, int6
   }
   const int64_t rg_per_wg = p.skinny ? kFwdSkinnyRG : (w8 ? wrg : wide_rg(w->type));
   const int64_t gx = cdiv(w->Np / 16, rg_per_wg);
-  // the large-grid kernel once its 128 x 128 tiles alone give a workgroup per CU, else its
-  // 128 x 64 tiles if those do
+  // the large-grid kernels (tiles of 128 rows x 128, 64 or 32 tokens; tokens < t only).  Automatic:
+  //  * the int8-MFMA form on 64-token tiles where those give 1.6 workgroups per CU (Q4_0: the f16 form on
+  //    128-token tiles from 16 of those per CU, and on rows of 256 columns from one); both forms agree bit for
+  //    bit without an adapter;
+  //  * else 32-token tiles where they give 1.5 workgroups per CU (below, the eight-wave tiles, which split
+  //    the columns over their waves, are as fast on long rows);
+  //  * else the eight-wave tiles.
+  // Measured per forward kernel, us, i8-64 / f16-128 / f16-32 / eight-wave: Q4_0 4096 x 1024 at 256, 512, 1001,
+  // 2048 tokens 17 / 23 / 13 / 18, 18 / 24 / 16 / 26, 22 / 26 / 28 / 49, 38 / 36 / 46 / 89; 6144 x 1024 at
+  // 1001, 2048 28 / 34 / 36 / 66, 50 / 53 / 66 / 129; 151936 x 1024 at 37, 256, 512 69 / 71 / 91 / 103,
+  // 140 / 151 / 203 / 396, 321 / 316 / 435 / 789; 1024 x 3072 at 1001, 2048 40 / 56 / 32 / 30, 42 / 58 / 37 /
+  // 46; Q8_0 14336 x 4096 at 100, 256, 2048 48 / 70 / 43 / 54, 60 / 76 / 78 / 91, 391 / 428 / 568 / 738.
+  // Rows of 256 columns, i8-64 / f16-128, 4096, 8192 and 16384 rows at 1024 tokens 11 / 13, 17.5 / 16.5,
+  // 27.6 / 28.0, at 2048 17.5 / 16.2, 27.2 / 28.1, 47 / 50 (of 512 columns, 4096 rows at 1024: 15 / 17.6)
   const int64_t mm_rows = cdiv(w->Np / 16, 8);
-  const int64_t mm128 = mm_rows * (p.Tp / kMmTile), mm64 = mm_rows * (p.Tp / 64), mm32 = mm_rows * (p.Tp / 32);
+  const int64_t mm128 = mm_rows * cdiv(t, kMmTile), mm64 = mm_rows * cdiv(t, 64), mm32 = mm_rows * cdiv(t, 32);
   int mm_ttn = 0;  // token tiles per workgroup of the chosen rtq_mm kernel, 0: none
-  if (!p.skinny && !isums && !is_kquant(w->type)) {
+  bool mmi8 = false;
+  if (!p.skinny && !isums && !kq) {
+    const int64_t cu = c->cu_count;
     if (c->fwd_mm == 1) mm_ttn = 8;
     else if (c->fwd_mm == 2) mm_ttn = 4;
     else if (c->fwd_mm == 3) mm_ttn = 2;
-    // automatic: 128-token tiles when they give every CU a workgroup; else 32-token tiles when 64-token
-    // ones would (two or more workgroups per CU hide the K loop's latencies better than one: 1.15
-    // against 1.27 ms per Qwen3-0.6B-shaped 512-token step over its q|k|v and gate|up products)
-    else if (c->fwd_mm < 0) mm_ttn = mm128 >= c->cu_count ? 8 : (mm64 >= c->cu_count ? 2 : 0);
+    else if (c->fwd_mm < 0) {
+      const bool q4_f16 = w->type == RTQ_TYPE_Q4_0 && (mm128 >= 16 * cu || (w->cols <= 256 && mm128 >= cu));
+      if (5 * mm64 >= 8 * cu) mm_ttn = q4_f16 ? 8 : 4;
+      else if (2 * mm32 >= 3 * cu) mm_ttn = 2;
+    }
+    // a Q4_0 weight's 64-token tiles asked for by RTQ_FWD_MM stay the f16 kernel's
+    mmi8 = mm_ttn >= 4 && (c->fwd_i8 == 1 || (c->fwd_i8 < 0 && (w->type == RTQ_TYPE_Q8_0 || (c->fwd_mm < 0 && mm_ttn == 4))));
+    if (mmi8) mm_ttn = 4;
   }
   const bool mm = mm_ttn > 0;
-  // the int8-MFMA kernel where the 128- or 64-token tiles are chosen, on 64-token tiles (its 128-token
-  // form holds 300 VGPRs, one wave per SIMD).  Automatic: for Q8_0 weights, whose codes reach the
-  // i8 MFMA as they lie in LDS; measured per forward call (activation kernel included) at 2048
-  // tokens: LM head 151936 x 1024 980 against 1020 us (f16, 128-token tiles), 28672 x 4096 848
-  // against 897, 6144 x 4096 241 against 259 (f16, 64-token tiles); Q4_0 mixed (1043 against
-  // 1005 us on the LM head, 864 against 906 on 28672 x 4096), so Q4_0 keeps the f16 kernels.
-  // Both agree bit for bit without an adapter.
-  const bool mmi8 = mm && (mm_ttn == 8 || mm_ttn == 4) &&
-                    (c->fwd_i8 == 1 || (c->fwd_i8 < 0 && w->type == RTQ_TYPE_Q8_0));
-  if (mmi8) mm_ttn = 4;
   // K-quants: the LDS-ring kernel where its 128 x 64 tiles (of tokens < t) give half the CUs two workgroups,
   // else the tile kernel (rtq_fwd_*_w).  Measured per forward kernel, ring / tile, us (and workgroups):
   // Q4_K 9728 x 2560 at 200, 400, 1001 tokens 49 / 42 (304), 64 / 70 (532), 108 / 147 (1216); Q6_K 2560 x

@@ -14,7 +14,8 @@ import rust_trainer_amd as rt
 
 pytestmark = pytest.mark.gpu
 
-KNOBS = {"mmk": {"RTQ_FWD_MMK": "1"}, "auto": {}}
+KNOBS = {"mm128": {"RTQ_FWD_MM": "1", "RTQ_FWD_I8": "0"}, "mm64": {"RTQ_FWD_MM": "2", "RTQ_FWD_I8": "0"},
+         "mm32": {"RTQ_FWD_MM": "3"}, "i8": {"RTQ_FWD_MM": "2", "RTQ_FWD_I8": "1"}, "mmk": {"RTQ_FWD_MMK": "1"}, "auto": {}}
 
 
 @pytest.fixture(scope="module", params=list(KNOBS))
