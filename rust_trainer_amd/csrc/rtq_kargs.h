@@ -100,8 +100,8 @@ struct ActArgs {
 
 // ---------------------------------------------------------------- trainer-native weights
 // FrozenWeight::{F32, Q8_0} (src/frozen.rs:33-45): f32 [N][K], or f32 scales [N][K/32] then i8
-// codes [N][K] (TQ8_0).  Their products run on the f32 MFMA GEMM (rtq_m_gemm*, the TQ8_0 codes
-// decoded in its operand loads); these kernels dequantise rows (out = 0 + d * q, row() of
+// codes [N][K] (TQ8_0).  Their products run on rtq_dense_fwd* / rtq_dense_bwd* or the f32 MFMA
+// GEMM (rtq_m_gemm*, the TQ8_0 codes decoded in its operand loads); these kernels dequantise rows (out = 0 + d * q, row() of
 // src/frozen.rs:172-176), copy rows and add the bias.
 struct DenseArgs {
   const float* w;    // F32 weight, or null

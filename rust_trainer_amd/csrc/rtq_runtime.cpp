@@ -353,7 +353,7 @@ rtq_status ensure_ws(rtq_ctx* c, size_t bytes) {
 
 bool is_q32(int type) { return type == RTQ_TYPE_Q4_0 || type == RTQ_TYPE_Q8_0; }
 bool is_kquant(int type) { return type == RTQ_TYPE_Q4_K || type == RTQ_TYPE_Q6_K; }
-// trainer-native FrozenWeight storage: f32 products on the f32 MFMA GEMM
+// trainer-native FrozenWeight storage: f32 products on split bf16 MFMAs (rtq_dense_*) or the f32 MFMA GEMM
 bool is_dense(int type) { return type == RTQ_TYPE_F32 || type == RTQ_TYPE_TQ8_0; }
 bool supported(int type) { return is_q32(type) || is_kquant(type) || is_dense(type); }
 int fmt_index(int type) {
@@ -494,8 +494,8 @@ size_t fwd_ws_bytes(const FwdPlan& p) {
 
 // ------------------------------------------------------------------ trainer-native weights
 // FrozenWeight::{F32, Q8_0} (src/frozen.rs:33-187) and the Linear LoRA math around them as f32
-// products on the f32 MFMA GEMM of the decoder kernels (rtq_m_gemm*: exact f32 products, f32
-// accumulation).  A TQ8_0 weight is read as codes plus one f32 scale per 32 and decoded in the
+// products on rtq_dense_* (see dense_fast), else on the f32 MFMA GEMM of the decoder kernels
+// (rtq_m_gemm*: exact f32 products, f32 accumulation).  A TQ8_0 weight is read as codes plus one f32 scale per 32 and decoded in the
 // GEMM's operand loads: no dequantised copy of the weight is materialised.
 
 // C(m, n) (+)= sum_k A(m, k) B(k, n), A(m, k) = a_scale * A[m * sAm + k * sAk] (the product rounded
@@ -1365,13 +1365,19 @@ rtq_status rtq_ctx_reserve(rtq_ctx* c, int64_t max_t, int64_t max_rows, int64_t 
   fake.Kp = roundup(max_cols, RTQ_CHUNK_Q);
   fake.type = RTQ_TYPE_Q4_0;
   size_t need = fwd_ws_bytes(fwd_plan(&fake, max_t, max_rank));
-  // the dx plans' split tiles: fewer tokens can need more of them
+  // the dx plans' split tiles: fewer tokens or a narrower weight can need more of them
+  const int64_t step = std::max<int64_t>(64, roundup(cdiv(max_t, 1024), 64));
   for (int type : {RTQ_TYPE_Q4_0, RTQ_TYPE_Q4_K}) {
     fake.type = type;
-    const int64_t step = std::max<int64_t>(64, roundup(cdiv(max_t, 1024), 64));
-    for (int64_t t = 64; t < max_t; t += step) need = std::max(need, bwd_ws_bytes(c, &fake, t, max_rank));
-    for (int64_t t : {std::min<int64_t>(max_t, 16), max_t}) need = std::max(need, bwd_ws_bytes(c, &fake, t, max_rank));
+    for (int64_t k = max_cols; k > 0; k -= 512) {
+      fake.cols = k;
+      fake.Kp = roundup(k, RTQ_CHUNK_Q);
+      for (int64_t t = 64; t < max_t; t += step) need = std::max(need, bwd_ws_bytes(c, &fake, t, max_rank));
+      for (int64_t t : {std::min<int64_t>(max_t, 16), max_t}) need = std::max(need, bwd_ws_bytes(c, &fake, t, max_rank));
+    }
   }
+  fake.cols = max_cols;
+  fake.Kp = roundup(max_cols, RTQ_CHUNK_Q);
   fake.type = RTQ_TYPE_F32;
   need = std::max({need, fwd_ws_bytes(fwd_plan(&fake, max_t, max_rank)), bwd_ws_bytes(c, &fake, max_t, max_rank)});
   RTQ_TRY(ensure_ws(c, need));
