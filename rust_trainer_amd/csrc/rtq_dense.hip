@@ -6,11 +6,15 @@
 //   rtq_dense_bwd32 / 64[_q8]:  part[z][t][k] = sum over the rows n of split z of dy[t][n] W[n][k]
 //     (rtq_bwd_finish sums the splits in order), or dx itself when there is one split and no adapter.
 //
-// An f32 value is exactly the sum of three bf16 values (each the truncation of what is left), so a
-// product is six bf16 MFMAs (hi hi | hi mid, mid hi, mid mid, hi lo, lo hi; the three terms left out
-// are below 2^-24 of the product, the rounding of an f32 product) at 16 times the f32 MFMA's rate.
+// An f32 value is exactly the sum of three bf16 values (each the truncation of what is left: mid is below
+// 2^-7 of the value's leading bit, lo below 2^-15), so a product is eight bf16 MFMAs (all pairs of planes but
+// lo lo, below 2^-30 of the product, a fraction of an f32 rounding) at 16 times the f32 MFMA's rate.  Without
+// mid lo and lo mid a product lost up to 2^-21, always in its own sign: a sum of one or a few large terms was
+// off by up to 3.5e-7 where f32 products leave 6e-8.
 // hi hi and the corrections accumulate apart.  The forward of codes needs three: a code is one exact
-// bf16 value, and a 32-element step is one scale's block, whose sum is scaled once (f32 FMA).
+// bf16 value, and a 32-element step is one scale's block, whose sum is scaled once (f32 FMA).  Its hi part and
+// the rest meet in an f32 add: the MFMA's own sum of the two is not rounded to nearest (a product of one term
+// was off by up to 2.4 2^-24 instead of 2 2^-24).
 // bf16 keeps f32's exponent range, so no operand is scaled.  An infinite or NaN operand turns the split
 // sums into NaN: such an output is summed again in plain f32 (dense_slow), which keeps the infinities.
 //
@@ -24,7 +28,8 @@
 // apart, and the eight rows of a wave's load are 4 apart (two sets): reads and writes then meet every
 // bank once (a 16-byte access serves lanes 0-3, 12-15, 20-23, 24-27 together, an 8-byte one a half-wave).
 // Measured, TQ8_0 2048 x 1024, 300 tokens, forward + backward with a rank-8 adapter, whole call: 317 us
-// on the f32 MFMA GEMM with one launch per adapter product, 60 here (forward kernel 21, backward 24);
+// on the f32 MFMA GEMM with one launch per adapter product, 61 here (six products: 59; 4096 x 4096, 1024 tokens,
+// backward 327 against 300);
 // against float64 1e-6 there, 2.2e-7 here.  Bound by the wait of each step (one barrier, LDS and MFMA
 // latency) at small grids, by MFMA (38% busy) and LDS (48%) at large ones.
 #define DENSE_D 4
@@ -221,9 +226,9 @@ __device__ __forceinline__ void dense_tile(const DenseGemmArgs& a) {
   };
   auto compute = [&](const Frags& F) {
     if constexpr (CODES) {
-      f4 b[WT][WC];
+      f4 b[WT][WC], hi[WT][WC];
 #pragma unroll
-      for (int p = 2; p >= 0; p--)
+      for (int p = 2; p >= 1; p--)
 #pragma unroll
         for (int j = 0; j < WC; j++)
 #pragma unroll
@@ -231,13 +236,17 @@ __device__ __forceinline__ void dense_tile(const DenseGemmArgs& a) {
 #pragma unroll
       for (int j = 0; j < WC; j++)
 #pragma unroll
+        for (int i = 0; i < WT; i++) hi[i][j] = mfma_bf16(F.w[j][0], F.x[i][0], f4{0.0f, 0.0f, 0.0f, 0.0f});
+#pragma unroll
+      for (int j = 0; j < WC; j++)
+#pragma unroll
         for (int i = 0; i < WT; i++)
 #pragma unroll
-          for (int e = 0; e < 4; e++) acc[i][j][e] = fmaf(F.d[j][e], b[i][j][e], acc[i][j][e]);
+          for (int e = 0; e < 4; e++) acc[i][j][e] = fmaf(F.d[j][e], hi[i][j][e] + b[i][j][e], acc[i][j][e]);
     } else {
-      constexpr int PA[5] = {2, 0, 1, 1, 0}, PB[5] = {0, 2, 1, 0, 1};
+      constexpr int PA[7] = {2, 1, 2, 0, 1, 1, 0}, PB[7] = {1, 2, 0, 2, 1, 0, 1};
 #pragma unroll
-      for (int p = 0; p < 5; p++)
+      for (int p = 0; p < 7; p++)
 #pragma unroll
         for (int j = 0; j < WC; j++)
 #pragma unroll

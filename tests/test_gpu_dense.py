@@ -2,8 +2,8 @@
 their tiles: one token, 31 / 32 / 33 and 64 / 65 tokens, rows that leave a tile or a 32-row step ragged,
 a row count that is no multiple of 4 (scalar dy loads), one 32-column block, enough tiles for the
 64-token form, several row splits.  An f32 dot of n terms is within (n / 2 + 2) 2^-24 of the sum of its
-terms' magnitudes however it is ordered; the products here leave out terms below 2^-24 each, so the
-bound below is (n / 16 + 4) 2^-24 of that sum (a rounding per 32-element step and the split's remainder)."""
+terms' magnitudes however it is ordered; the products here leave out terms below 2^-30 each, so the
+bound below is (n / 16 + 4) 2^-24 of that sum (a rounding per 32-element step and of the split's parts)."""
 import numpy as np
 import pytest
 
@@ -83,3 +83,26 @@ def test_dense_products_keep_infinities(ctx, kind):
             inf = np.isinf(want)
             assert np.array_equal(got[inf], want[inf].astype(np.float32))
             assert np.isfinite(got[np.isfinite(want)]).all()
+
+
+@pytest.mark.parametrize("kind", ["f32", "tq8"])
+@pytest.mark.parametrize("n,k,t", [(65, 64, 33), (1030, 2048, 65)])
+def test_dense_products_of_single_terms(ctx, kind, n, k, t):
+    """Rows with one non-zero element, as masked gradients have: each output is one product, so nothing averages
+    out what the split leaves behind.  An f32 product is off by at most 2^-24; here the corrections' sum, up to
+    2^-6 of the product, is rounded seven times more, which is 2^-24 (1 + 7 / 64).  TQ8_0's forward rounds the
+    product with the code, then that with the scale, and the corrections twice."""
+    hw, w = _weight(ctx, kind, n, k)
+    r = np.random.RandomState(1)
+    x, dy = np.zeros((t, k), np.float32), np.zeros((t, n), np.float32)
+    xc, dc = r.randint(0, k, t), r.randint(0, n, t)
+    x[np.arange(t), xc] = np.exp(r.randn(t))
+    dy[np.arange(t), dc] = -np.exp(3 * r.randn(t))
+    eps = 2.0 ** -24
+    y = hw.forward(x, t).reshape(t, n)
+    want = x[np.arange(t), xc].astype(np.float64)[:, None] * w[:, xc].T
+    assert (np.abs(y - want) <= (2.125 if kind == "tq8" else 1.125) * eps * np.abs(want)).all()
+    dx = np.zeros(t * k, np.float32)
+    hw.backward_input(dy, t, dx)
+    want = dy[np.arange(t), dc].astype(np.float64)[:, None] * w.astype(np.float32)[dc]  # codes decoded to f32
+    assert (np.abs(dx.reshape(t, k) - want) <= 1.125 * eps * np.abs(want)).all()
