@@ -16,7 +16,7 @@
 // the rest meet in an f32 add: the MFMA's own sum of the two is not rounded to nearest (a product of one term
 // was off by up to 2.4 2^-24 instead of 2 2^-24).
 // bf16 keeps f32's exponent range, so no operand is scaled.  An infinite or NaN operand turns the split
-// sums into NaN: such an output is summed again in plain f32 (dense_slow), which keeps the infinities.
+// sums into NaN: such an output is summed again on the f32 MFMA, which keeps the infinities.
 //
 // Workgroup: four waves, 64 weight-side outputs x 16 TT tokens (TT = 4: wave (w % 2, w / 2) takes 32 x
 // 32; TT = 2: wave w takes 16 x 32).  Per 32-element step the operands go global -> registers (D - 1
@@ -52,20 +52,6 @@ __device__ __forceinline__ void split3(float a, float b, uint32_t& h, uint32_t& 
   m = __builtin_amdgcn_perm(vb, va, 0x07060302u);
   const float sa = ra - __uint_as_float(va & 0xffff0000u), sb = rb - __uint_as_float(vb & 0xffff0000u);
   l = __builtin_amdgcn_perm(__float_as_uint(sb), __float_as_uint(sa), 0x07060302u);
-}
-
-// element (n, k) of the weight in f32 (0 + d * q, src/frozen.rs:172-176)
-template <bool Q8>
-__device__ __forceinline__ float dense_w(const DenseGemmArgs& a, int n, int k) {
-  if (Q8) return a.sc[(int64_t)n * (a.K / 32) + (k >> 5)] * (float)a.qs[(int64_t)n * a.K + k];
-  return a.w[(int64_t)n * a.K + k];
-}
-template <bool BWD, bool Q8>
-__device__ __forceinline__ float dense_slow(const DenseGemmArgs& a, int t, int o, int c0, int c1) {
-  float s = 0.0f;
-  const int C = BWD ? a.N : a.K;
-  for (int c = c0; c < c1; c++) s = fmaf(a.x[(int64_t)t * C + c], BWD ? dense_w<Q8>(a, c, o) : dense_w<Q8>(a, o, c), s);
-  return s;
 }
 
 template <bool BWD, bool Q8, int TT>
@@ -284,17 +270,61 @@ __device__ __forceinline__ void dense_tile(const DenseGemmArgs& a) {
 #pragma unroll
     for (int v = 0; v < D; v++) step_body(v, nfull + v, false);
   }
+  bool again = false;
 #pragma unroll
   for (int i = 0; i < WT; i++)
 #pragma unroll
     for (int j = 0; j < WC; j++) {
       acc[i][j] += low[i][j];
 #pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const int t = t0 + 16 * (wt + i) + li, o = o0 + 16 * (wc + j) + 4 * g + e;
-        if (acc[i][j][e] != acc[i][j][e] && t < a.T && o < O) acc[i][j][e] = dense_slow<BWD, Q8>(a, t, o, c0, c1);
-      }
+      for (int e = 0; e < 4; e++) again |= acc[i][j][e] != acc[i][j][e];
     }
+  // A wave with a NaN sums its tiles once more on the f32 MFMA (the operands straight from memory; a step of 16
+  // elements, k-group g taking 4 g .. + 3) and takes those of its NaN outputs.  One lane per output took some
+  // hundred times as long where a whole activation is NaN
+  if (__ballot(again) != 0) {
+    f4 full[WT][WC];
+#pragma unroll
+    for (int i = 0; i < WT; i++)
+#pragma unroll
+      for (int j = 0; j < WC; j++) full[i][j] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int c = c0; c < c1; c += 16) {
+      f4 xv[WT], wv[WC];
+#pragma unroll
+      for (int i = 0; i < WT; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const uint32_t o = ((uint32_t)min(t0 + 16 * (wt + i) + li, a.T) * C + 4 * g + e) * 4u;
+          const float v = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, o, (uint32_t)c * 4u, 0));
+          xv[i][e] = c + 4 * g + e < C ? v : 0.0f;  // elements past C hold the next row's
+        }
+#pragma unroll
+      for (int j = 0; j < WC; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const int o = o0 + 16 * (wc + j) + li, ce = c + 4 * g + e;
+          const uint32_t n = min(BWD ? ce : o, a.N), k = BWD ? min(o, a.K - 1) : ce;  // row N: past the end, zeros
+          if constexpr (Q8) {
+            const int q = (int8_t)__builtin_amdgcn_raw_buffer_load_b8(rw, n * a.K + k, 0, 0);
+            wv[j][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, (n * (a.K / 32) + (k >> 5)) * 4u, 0, 0)) * (float)q;
+          } else {
+            wv[j][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rw, (n * a.K + k) * 4u, 0, 0));
+          }
+        }
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+#pragma unroll
+        for (int i = 0; i < WT; i++)
+#pragma unroll
+          for (int j = 0; j < WC; j++) full[i][j] = mfma_f32(wv[j][e], xv[i][e], full[i][j]);
+    }
+#pragma unroll
+    for (int i = 0; i < WT; i++)
+#pragma unroll
+      for (int j = 0; j < WC; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[i][j][e] = acc[i][j][e] != acc[i][j][e] ? full[i][j][e] : acc[i][j][e];
+  }
 
   // the adapter's part, 32 ranks at a time: forward s h B^T, h summed from its slice partials; backward
   // (the first split) g A, g likewise

@@ -106,3 +106,30 @@ def test_dense_products_of_single_terms(ctx, kind, n, k, t):
     hw.backward_input(dy, t, dx)
     want = dy[np.arange(t), dc].astype(np.float64)[:, None] * w.astype(np.float32)[dc]  # codes decoded to f32
     assert (np.abs(dx.reshape(t, k) - want) <= 1.125 * eps * np.abs(want)).all()
+
+
+@pytest.mark.parametrize("kind", ["f32", "tq8"])
+def test_dense_products_of_nan_rows_take_their_time(ctx, kind):
+    """A diverged run's NaN activations and gradients: their products are NaN, by the second sum that keeps
+    infinities apart, at a small multiple of the ordinary time (the second sum runs on the f32 MFMA, a sixteenth
+    of the bf16 one's rate, without the first one's staging)."""
+    n, k, t = 1024, 1024, 512
+    hw, _ = _weight(ctx, kind, n, k)
+
+    def ms(x):
+        ctx.set_timing(True)
+        ctx.reset_timing()
+        for _ in range(3):
+            out = hw.forward(x, t)
+            hw.backward_input(x, t, np.zeros(t * k, np.float32))
+        ran = {name: v for name, v in ctx.timing().items() if name.startswith("rtq_dense")}
+        ctx.set_timing(False)
+        assert len(ran) == 2, ran
+        return sum(v[1] for v in ran.values()), out
+
+    x = O.Rng(2).vec_normal(t * k, 1.0)
+    ms(x)
+    plain, _ = ms(x)
+    slow, out = ms(np.full(t * k, np.nan, np.float32))
+    assert np.isnan(out).all()
+    assert slow <= 20 * plain, (slow, plain)
