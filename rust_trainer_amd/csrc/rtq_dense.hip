@@ -16,7 +16,8 @@
 // the rest meet in an f32 add: the MFMA's own sum of the two is not rounded to nearest (a product of one term
 // was off by up to 2.4 2^-24 instead of 2 2^-24).
 // bf16 keeps f32's exponent range, so no operand is scaled.  An infinite or NaN operand turns the split
-// sums into NaN: such an output is summed again on the f32 MFMA, which keeps the infinities.
+// sums into NaN, and an unscaled sum of codes can overflow where the scaled one does not: an output that is
+// not finite is summed again on the f32 MFMA.
 //
 // Workgroup: four waves, 64 weight-side outputs x 16 TT tokens (TT = 4: wave (w % 2, w / 2) takes 32 x
 // 32; TT = 2: wave w takes 16 x 32).  Per 32-element step the operands go global -> registers (D - 1
@@ -53,6 +54,8 @@ __device__ __forceinline__ void split3(float a, float b, uint32_t& h, uint32_t& 
   const float sa = ra - __uint_as_float(va & 0xffff0000u), sb = rb - __uint_as_float(vb & 0xffff0000u);
   l = __builtin_amdgcn_perm(__float_as_uint(sb), __float_as_uint(sa), 0x07060302u);
 }
+
+__device__ __forceinline__ bool dense_again(float v) { return !(fabsf(v) < INFINITY); }
 
 template <bool BWD, bool Q8, int TT>
 __device__ __forceinline__ void dense_tile(const DenseGemmArgs& a) {
@@ -277,10 +280,10 @@ __device__ __forceinline__ void dense_tile(const DenseGemmArgs& a) {
     for (int j = 0; j < WC; j++) {
       acc[i][j] += low[i][j];
 #pragma unroll
-      for (int e = 0; e < 4; e++) again |= acc[i][j][e] != acc[i][j][e];
+      for (int e = 0; e < 4; e++) again |= dense_again(acc[i][j][e]);
     }
-  // A wave with a NaN sums its tiles once more on the f32 MFMA (the operands straight from memory; a step of 16
-  // elements, k-group g taking 4 g .. + 3) and takes those of its NaN outputs.  One lane per output took some
+  // A wave with such an output sums its tiles once more on the f32 MFMA (the operands straight from memory; a step
+  // of 16 elements, k-group g taking 4 g .. + 3) and takes those outputs.  One lane per output took some
   // hundred times as long where a whole activation is NaN
   if (__ballot(again) != 0) {
     f4 full[WT][WC];
@@ -323,7 +326,7 @@ __device__ __forceinline__ void dense_tile(const DenseGemmArgs& a) {
 #pragma unroll
       for (int j = 0; j < WC; j++)
 #pragma unroll
-        for (int e = 0; e < 4; e++) acc[i][j][e] = acc[i][j][e] != acc[i][j][e] ? full[i][j][e] : acc[i][j][e];
+        for (int e = 0; e < 4; e++) acc[i][j][e] = dense_again(acc[i][j][e]) ? full[i][j][e] : acc[i][j][e];
   }
 
   // the adapter's part, 32 ranks at a time: forward s h B^T, h summed from its slice partials; backward

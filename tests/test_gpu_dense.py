@@ -133,3 +133,21 @@ def test_dense_products_of_nan_rows_take_their_time(ctx, kind):
     slow, out = ms(np.full(t * k, np.nan, np.float32))
     assert np.isnan(out).all()
     assert slow <= 20 * plain, (slow, plain)
+
+
+@pytest.mark.parametrize("kind", ["f32", "tq8"])
+def test_dense_products_of_large_values(ctx, kind):
+    """Operands near the top of f32's range whose products with the weight are far from it: a block's sum with
+    the codes (up to 127) overflows before its scale (here about 5e-4) brings it back."""
+    n, k, t = 70, 64, 40
+    hw, w = _weight(ctx, kind, n, k)
+    x = O.Rng(2).vec_normal(t * k, 1e37).reshape(t, k)
+    x[3, 5] = 3.4e38
+    x[4] = np.where(w[0] < 0, -2e36, 2e36)  # no product with a code overflows, their sum does
+    dy = O.Rng(3).vec_normal(t * n, 1e37).reshape(t, n)
+    dx = np.zeros(t * k, np.float32)
+    hw.backward_input(dy, t, dx)
+    for got, a, b in ((hw.forward(x, t), x.astype(np.float64), w.T), (dx, dy.astype(np.float64), w)):
+        want, size = a @ b, np.abs(a) @ np.abs(b)
+        assert np.abs(want).max() < 1e38
+        assert (np.abs(got.reshape(want.shape).astype(np.float64) - want) <= (b.shape[0] / 16 + 4) * 2.0 ** -24 * size).all()
