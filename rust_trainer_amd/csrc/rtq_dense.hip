@@ -15,9 +15,14 @@
 // bf16 value, and a 32-element step is one scale's block, whose sum is scaled once (f32 FMA).  Its hi part and
 // the rest meet in an f32 add: the MFMA's own sum of the two is not rounded to nearest (a product of one term
 // was off by up to 2.4 2^-24 instead of 2 2^-24).
-// bf16 keeps f32's exponent range, so no operand is scaled.  An infinite or NaN operand turns the split
+// bf16 keeps f32's exponent range, so no operand is scaled.  But the bf16 MFMA takes a denormal operand or
+// product as zero: below about 2^-110 a value loses its lo plane, and products below 2^-100 their corrections
+// (1e-34 times 0.02 was off by up to 3000 2^-24).  What is lost is below 2^-126 a term, so an output of 2^-80
+// or more does not notice, and a smaller one is summed again on the f32 MFMA.  (An output below the least
+// normal value can come out as 0.)  An infinite or NaN operand turns the split
 // sums into NaN, and an unscaled sum of codes can overflow where the scaled one does not: an output that is
-// not finite is summed again on the f32 MFMA.
+// not finite is summed again too.  1024 x 1024, 512 tokens, all outputs summed again: 82 us a forward product
+// against 20, 108 against 18 for TQ8_0.
 //
 // Workgroup: four waves, 64 weight-side outputs x 16 TT tokens (TT = 4: wave (w % 2, w / 2) takes 32 x
 // 32; TT = 2: wave w takes 16 x 32).  Per 32-element step the operands go global -> registers (D - 1
@@ -55,7 +60,10 @@ __device__ __forceinline__ void split3(float a, float b, uint32_t& h, uint32_t& 
   l = __builtin_amdgcn_perm(__float_as_uint(sb), __float_as_uint(sa), 0x07060302u);
 }
 
-__device__ __forceinline__ bool dense_again(float v) { return !(fabsf(v) < INFINITY); }
+__device__ __forceinline__ bool dense_again(float v) {
+  const float m = fabsf(v);
+  return !(m < INFINITY) || (m > 0.0f && m < 0x1p-80f);
+}
 
 template <bool BWD, bool Q8, int TT>
 __device__ __forceinline__ void dense_tile(const DenseGemmArgs& a) {

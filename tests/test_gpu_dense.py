@@ -87,25 +87,27 @@ def test_dense_products_keep_infinities(ctx, kind):
 
 @pytest.mark.parametrize("kind", ["f32", "tq8"])
 @pytest.mark.parametrize("n,k,t", [(65, 64, 33), (1030, 2048, 65)])
-def test_dense_products_of_single_terms(ctx, kind, n, k, t):
+@pytest.mark.parametrize("unit", [0, -112, -118])
+def test_dense_products_of_single_terms(ctx, kind, n, k, t, unit):
     """Rows with one non-zero element, as masked gradients have: each output is one product, so nothing averages
     out what the split leaves behind.  An f32 product is off by at most 2^-24; here the corrections' sum, up to
     2^-6 of the product, is rounded seven times more, which is 2^-24 (1 + 7 / 64).  TQ8_0's forward rounds the
-    product with the code, then that with the scale, and the corrections twice."""
+    product with the code, then that with the scale, and the corrections twice.  Small values (2^unit), whose planes
+    or products are denormal, keep that; an output below the least normal value may be zero."""
     hw, w = _weight(ctx, kind, n, k)
     r = np.random.RandomState(1)
     x, dy = np.zeros((t, k), np.float32), np.zeros((t, n), np.float32)
     xc, dc = r.randint(0, k, t), r.randint(0, n, t)
-    x[np.arange(t), xc] = np.exp(r.randn(t))
-    dy[np.arange(t), dc] = -np.exp(3 * r.randn(t))
+    x[np.arange(t), xc] = np.exp(r.randn(t)) * 2.0 ** unit
+    dy[np.arange(t), dc] = -np.exp(3 * r.randn(t)) * 2.0 ** unit
     eps = 2.0 ** -24
     y = hw.forward(x, t).reshape(t, n)
     want = x[np.arange(t), xc].astype(np.float64)[:, None] * w[:, xc].T
-    assert (np.abs(y - want) <= (2.125 if kind == "tq8" else 1.125) * eps * np.abs(want)).all()
+    assert (np.abs(y - want) <= (2.125 if kind == "tq8" else 1.125) * eps * np.abs(want) + 2.0 ** -126).all()
     dx = np.zeros(t * k, np.float32)
     hw.backward_input(dy, t, dx)
     want = dy[np.arange(t), dc].astype(np.float64)[:, None] * w.astype(np.float32)[dc]  # codes decoded to f32
-    assert (np.abs(dx.reshape(t, k) - want) <= 1.125 * eps * np.abs(want)).all()
+    assert (np.abs(dx.reshape(t, k) - want) <= 1.125 * eps * np.abs(want) + 2.0 ** -126).all()
 
 
 @pytest.mark.parametrize("kind", ["f32", "tq8"])
