@@ -687,6 +687,14 @@ __device__ __forceinline__ void act_prep(const ActArgs& a) {
     if (kk < a.Kp) {
       const int b = kk >> 5, hf = sg & 1, kc = b >> 2, j = b & 3;
       if (a.xq_i8) {  // uniform: int8 fragments of rtq_mmi8_*, k-group g at byte 8 (g % 2) + 4 hf of lane (t % 32) + 32 (g / 2)
+        // a NaN has no int8 code (it becomes 0): its block's scale carries it, as the f16 code does
+        if (!QK) {
+          float nan = 0.0f;
+#pragma unroll
+          for (int i = 0; i < 16; i++) nan = v[i] != v[i] ? v[i] : nan;
+          nan = nan + __shfl_xor(nan, 1);
+          dstore = nan != nan ? nan : dstore;
+        }
         uint32_t* xq = reinterpret_cast<uint32_t*>(a.xq) + ((((int64_t)(t >> 5) * Kc + kc) * 4 + j) * 64 + (t & 31)) * 4 + hf;
 #pragma unroll
         for (int g = 0; g < 4; g++) {

@@ -55,3 +55,23 @@ def test_forward_token_tiles(ctx, n, k, t):
         y = lin.forward(x, t).reshape(t, n)
         want = want + 2 * (x.astype(np.float64) @ a.T.astype(np.float64)) @ b.T.astype(np.float64)
         assert np.abs(y - want).max() <= 2e-6 * np.abs(want).max(), wtype
+
+
+def test_forward_nan_rows(ctx):
+    """A token with a NaN gives NaN for every output on every kernel of the Q8_0 activations, the int8 ones too (a
+    NaN has no code there), and leaves the other tokens as they were.  (Q8_K's quantiser caps a code at 127, a NaN
+    among them.)"""
+    n, k, t = 130, 512, 70
+    formats = set(ctx.formats) & {O.Q4_0, O.Q8_0}
+    if not formats:
+        pytest.skip("no Q8_0 activations on this kernel")
+    for wtype in formats:
+        blocks = O.quantize(wtype, O.Rng(1).vec_normal(n * k, 0.02).reshape(n, k))
+        w = rt.HipFrozen(wtype, blocks, n, k, ctx=ctx)
+        x = O.Rng(2).vec_normal(t * k, 1.0).reshape(t, k)
+        plain = w.forward(x, t).reshape(t, n)
+        x[3, 100], x[66] = np.nan, np.nan
+        y = w.forward(x, t).reshape(t, n)
+        bad = np.isin(np.arange(t), (3, 66))
+        assert np.isnan(y[bad]).all(), wtype
+        assert np.array_equal(y[~bad], plain[~bad]), wtype
