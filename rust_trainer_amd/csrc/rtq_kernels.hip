@@ -2810,9 +2810,9 @@ extern "C" __global__ __launch_bounds__(256) void rtq_bwd_prep(BwdPrepArgs a) {
 // 32 columns (2 x 2 MFMA tiles).  Rows of W are split over workgroups; each split writes its own
 // partial tile (plain stores; rtq_bwd_finish sums the splits in order).  Per 32-row step the
 // workgroup stages, double buffered in LDS, f16 hi / lo MFMA operands:
-//   * dy[64 x 32]: each thread loads one float4, scales it by 2^e (e per token row and split, so
-//     that the split's largest |dy| of the row lands in [2^14, 2^15): the f16 range holds every
-//     value of the row) and splits it into hi = f16 (round toward zero) and lo = f16 of the rest;
+//   * dy[64 x 32]: each thread loads one float4, scales it by 2^e (e per token row and workgroup, so
+//     that the largest |dy| of the row in its rows lands in [2^14, 2^15); per range of 256 or 480 rows
+//     where a row's slices differ too much for one) and splits it into hi = f16 (round toward zero) and lo = f16 of the rest;
 //   * W[32 x 128]: Q4_0 / Q8_0 d * q exactly as hi = f16(d * q) and lo = d * q - hi (packed f16
 //     multiply and fused multiply-add on the two rows a thread converts: the residual of an f16
 //     product is exact); K-quants: the f32 value of ggml's dequantisation ((d*sc)*u - dmin*m, or
@@ -2920,7 +2920,6 @@ __device__ __forceinline__ void dx_tile(const DxArgs& a) {
   constexpr int D = TW == 64 ? 4 : 3;
   __shared__ u4v sA[2][TW / 16][2][64];                               // [buf][tile][hi/lo][lane]
   __shared__ __attribute__((aligned(16))) _Float16 sW[2][2][128][32];   // [buf][hi/lo][k][n], swizzled
-  __shared__ float sInv[TW];  // 2^-e (times wunsc) of each token row of the tile
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, li = lane & 15, g = lane >> 4;
   const int wt = TW == 64 ? w >> 2 : w >> 1, wk = TW == 64 ? w & 3 : w & 1;
   int tile, sp = 0, n0 = 0, n_len = a.Np;
@@ -2947,7 +2946,8 @@ __device__ __forceinline__ void dx_tile(const DxArgs& a) {
   // dy loader: tokens tl + 64 m (m < NQ), float4 q4 (columns ns + 4 q4 .. +3 of the step); eight
   // consecutive lanes take a row's 128 bytes (one or two L1 lines), and a wave's eight rows are 4 apart
   // (two sets), so that its 8-byte LDS writes at slot (row ^ q4 / 2) + 16 (q4 / 2) meet every bank once
-  const int wv = tid >> 6, tl = 16 * (wv >> 1) + 2 * (wv & 1) + 4 * ((lane >> 3) & 3) + (lane >> 5), q4 = lane & 7;
+  auto dy_row = [](int tid) { return 16 * (tid >> 7) + 2 * ((tid >> 6) & 1) + 4 * ((tid >> 3) & 3) + ((tid >> 5) & 1); };
+  const int tl = dy_row(tid), q4 = lane & 7;
   const __amdgpu_buffer_rsrc_t rdy = make_rsrc(a.dy, (uint32_t)a.T * a.N * 4u);
   const uint32_t dy_off = ((uint32_t)(t0 + tl) * a.N + 4 * q4) * 4u;
   const bool dy_vec = (a.N & 3) == 0;
@@ -2977,37 +2977,87 @@ __device__ __forceinline__ void dx_tile(const DxArgs& a) {
   const uint32_t q_rg = (uint32_t)Kc * 64 * 16 * (B8 ? 2 : 1);  // bytes per row group
   const uint32_t d_rg = (uint32_t)Kc * 128, e_rg = (uint32_t)Kc * 32;
 
-  // 2^e of this thread's dy rows tl + 64 m: e from the largest |dy| of the row over the slices of
-  // 256 rows that meet this split (their maxima from rtq_bwd_prep); 1 for a zero row.  All threads
-  // reduce the tile's rows: thread (row tid % TW, slices tid / TW + k (512 / TW)), then the partial
-  // maxima in LDS (a split may span many slices: 76 for a 19456-row weight).
+  // 2^e of this thread's dy rows tl + 64 m, e from the largest |dy| of the row over the slices of 256 rows
+  // that meet this workgroup's rows (their maxima from rtq_bwd_prep).  A row with a slice 2^18 or more below
+  // that would keep less of it than the products do (values 2^-39 below the range's top are lost, so 2^-21 of
+  // such a slice's own largest): then (segd, uniform) every token takes a range of its own per SEG steps and
+  // the sums are rescaled in between, exactly, by powers of two.
+  constexpr int SEG = TW == 64 ? 8 : 15;  // a multiple of D; 256 and 480 rows
+  constexpr int PER = 512 / TW;
+  __shared__ float2 sRed[512];  // (largest, least)
+  __shared__ float sScale[TW], sMin[TW], sMul[TW];  // 2^e, the least 2^e so far, the sums' factor at a change
+  __shared__ int sSeg;
   float dsc[NQ];
-  {
-    __shared__ float sRed[512];
-    constexpr int PER = 512 / TW;
-    const int q0 = n0 / 256, q1 = min((n0 + n_len + 255) / 256, a.dmq);
-    const int tok = tid % TW, t = t0 + tok;
-    float mx = 0.0f;
+  // the largest and the least non-zero maximum of row t0 + tid % TW over slices q0 .. q1 - 1, by all threads
+  // (slices tid / TW + k PER); the first TW threads return the rows' (a LM head's row spans 594 slices)
+  auto row_range = [&](int tid, int q0, int q1, float& mx, float& low) {
+    const int t = t0 + tid % TW;
+    mx = 0.0f;
+    low = INFINITY;
     if (t < a.T) {
 #pragma unroll 4
-      for (int q = q0 + tid / TW; q < q1; q += PER) mx = fmaxf(mx, a.dymax[(int64_t)q * a.T + t]);
+      for (int q = q0 + tid / TW; q < q1; q += PER) {
+        const float v = a.dymax[(int64_t)q * a.T + t];
+        mx = fmaxf(mx, v);
+        low = v > 0.0f ? fminf(low, v) : low;
+      }
     }
-    sRed[tid] = mx;
+    sRed[tid] = float2{mx, low};
     __syncthreads();
     if (tid < TW) {
-      float m = sRed[tid];
 #pragma unroll
-      for (int k = 1; k < PER; k++) m = fmaxf(m, sRed[tid + k * TW]);
-      int ex = 0;
-      (void)frexpf(m, &ex);  // m = f 2^ex, f in [0.5, 1)
-      const bool ok = m > 0.0f && m <= 3.0e38f;
-      sRed[tid] = ok ? ldexpf(1.0f, 15 - ex) : 1.0f;
-      sInv[tid] = (ok ? ldexpf(1.0f, ex - 15) : 1.0f) * a.wunsc;
+      for (int k = 1; k < PER; k++) {
+        const float2 o = sRed[tid + k * TW];
+        mx = fmaxf(mx, o.x);
+        low = fminf(low, o.y);
+      }
+    }
+  };
+  auto inverse = [](float p) { return __uint_as_float(0x7f000000u - __float_as_uint(p)); };  // of 2^e, |e| <= 126
+  // 2^(15 - ex) for m = f 2^ex, f in [0.5, 1); 0 for a zero or infinite m
+  auto scale_of = [](float m) {
+    int ex = 0;
+    (void)frexpf(m, &ex);
+    return m > 0.0f && m <= 3.0e38f ? ldexpf(1.0f, min(15 - ex, 126)) : 0.0f;
+  };
+  auto rows_of_steps = [&](int tid, int s, int e, float& mx, float& low) {
+    row_range(tid, (n0 + 32 * s) / 256, min((n0 + 32 * e + 255) / 256, a.dmq), mx, low);
+  };
+  bool segd;
+  {
+    if (tid == 0) sSeg = 0;
+    float mx, low;
+    rows_of_steps(tid, 0, nsteps, mx, low);
+    if (tid < TW) {
+      const float s = scale_of(mx);
+      sScale[tid] = sMin[tid] = s != 0.0f ? s : 1.0f;
+      if (s != 0.0f && low < mx * 3.814697265625e-6f) sSeg = 1;  // 2^-18
+    }
+    __syncthreads();
+    segd = sSeg != 0;
+  }
+  // the range of steps st ..: the token's own, or the present one where they hold zeros (or an infinity), and at
+  // most 2^60 times the widest one so far (sums of 2^48 at most then stay finite)
+  auto set_range = [&](int st) {
+    __syncthreads();
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));  // nothing of this is kept in registers over the main loop
+    float mx, low;
+    rows_of_steps(tid, st, min(st + SEG, nsteps), mx, low);
+    if (tid < TW) {
+      const float cur = sScale[tid], own = scale_of(mx), least = st == 0 ? 0x1p126f : sMin[tid];
+      const float s = own == 0.0f ? cur : fminf(own, least * 0x1p60f);
+      sMul[tid] = s * inverse(cur);
+      sMin[tid] = fminf(least, s);
+      sScale[tid] = s;
     }
     __syncthreads();
 #pragma unroll
-    for (int m = 0; m < NQ; m++) dsc[m] = sRed[tl + 64 * m];
-  }
+    for (int m = 0; m < NQ; m++) dsc[m] = sScale[dy_row(tid) + 64 * m];
+  };
+  if (segd) set_range(0);
+#pragma unroll
+  for (int m = 0; m < NQ; m++) dsc[m] = sScale[tl + 64 * m];
   // -1 as a run-time value (wsc * wunsc = 1 exactly), so v - hi stays one mixed-precision FMA
   const float neg1 = -(a.wsc * a.wunsc);
 
@@ -3039,7 +3089,7 @@ __device__ __forceinline__ void dx_tile(const DxArgs& a) {
   // The ragged tail of N (columns >= N of the last step hold the next row's values) is cleared here,
   // where the step's loads are consumed: clearing the load destinations right after issuing them
   // makes the compiler wait for every load in flight, the prefetched steps' included.
-  auto stage = [&](const DxSlot<FMT, NQ>& S, int buf, int step) {
+  auto stage_dy = [&](const DxSlot<FMT, NQ>& S, int buf, int step) {
     const int nst = n0 + 32 * min(step, max(nsteps - 1, 0));
 #pragma unroll
     for (int m = 0; m < NQ; m++) {  // dy: A fragment tile (tl>>4) + 4m, lane (tl&15) + 16*(q4>>1), slots 4*(q4&1) ..
@@ -3060,6 +3110,9 @@ __device__ __forceinline__ void dx_tile(const DxArgs& a) {
       reinterpret_cast<u2v*>(&sA[buf][(tl >> 4) + 4 * m][0][fl])[q4 & 1] = hv;
       reinterpret_cast<u2v*>(&sA[buf][(tl >> 4) + 4 * m][1][fl])[q4 & 1] = lv;
     }
+  };
+  auto stage = [&](const DxSlot<FMT, NQ>& S, int buf, int step) {
+    stage_dy(S, buf, step);
     // W: rows 2p, 2p+1 -> f16 hi / lo planes, one 32-bit word (both rows) per column
     uint32_t hw[4], lw[4];
     if constexpr (KQ) {
@@ -3164,25 +3217,36 @@ __device__ __forceinline__ void dx_tile(const DxArgs& a) {
     }
     __builtin_amdgcn_sched_barrier(0);
   };
+  // acc's rows times f: element i of acc[ts][ks] is tile row TW == 64 ? 32wt + 16ts + 4g + i : 64wt + 16ts + 4g + i
+  auto scale_rows = [&](auto f) {
+#pragma unroll
+    for (int ts = 0; ts < TS; ts++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const float sv = f((TW == 64 ? 32 : 64) * wt + 16 * ts + 4 * g + i);
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) acc[ts][ks][i] *= sv;
+      }
+  };
+  // before step st (a multiple of SEG): the next range; step st's dy is staged again in it (its buffer has no
+  // reader before the next barrier, and each thread writes the words that it wrote before)
+  auto next_range = [&](int st) {
+    set_range(st);
+    scale_rows([&](int row) { return sMul[row]; });
+    stage_dy(sl[0], st & 1, st);
+  };
   const int nfull = nsteps / D * D;
   for (int st0 = 0; st0 < nfull; st0 += D) {
+    if (segd && st0 > 0 && st0 % SEG == 0) next_range(st0);
 #pragma unroll
     for (int s0 = 0; s0 < D; s0++) step_body(s0, st0 + s0, true);
   }
   if (nfull < nsteps) {
+    if (segd && nfull > 0 && nfull % SEG == 0) next_range(nfull);
 #pragma unroll
     for (int s0 = 0; s0 < D; s0++) step_body(s0, nfull + s0, false);
   }
-  // rows back to dy's scale (and W's): element i of acc[ts][ks] is tile row TW == 64 ? 32wt + 16ts + 4g + i
-  // : 64wt + 16ts + 4g + i (sInv was written before the loop's first barrier)
-#pragma unroll
-  for (int ts = 0; ts < TS; ts++)
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const float sv = sInv[(TW == 64 ? 32 : 64) * wt + 16 * ts + 4 * g + i];
-#pragma unroll
-      for (int ks = 0; ks < KS; ks++) acc[ts][ks][i] *= sv;
-    }
+  scale_rows([&](int row) { return inverse(sScale[row]) * a.wunsc; });  // back to dy's scale, and W's
   // 64-token partial tiles in fragment order, [wave][q][lane] (float4 each), wave = 4 wt' + wk', q = 2 ts'
   // + ks' in the TW = 64 layout: element i is row 64 tile + 32wt' + 16ts' + 4g + i, column 128kc + 32wk' +
   // 16ks' + li.  Each 16-byte store of a wave writes 1 KB contiguously.  The first split of every tile at

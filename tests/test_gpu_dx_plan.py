@@ -54,3 +54,53 @@ def test_dx_split_tiles(ctx, wtype, n, k, t):
     got = lin.backward(x, dy, t).reshape(t, k)
     full = want + 2 * (dy.astype(np.float64) @ b) @ a.astype(np.float64)
     assert (np.abs(got - full) / np.abs(full).max(axis=1, keepdims=True)).max() <= 2e-6
+
+
+@pytest.fixture(scope="module", params=["0", "1"], ids=["tok64", "tok256"])
+def whole(request):
+    knobs = {"RTQ_DX_WIDE": request.param, "RTQ_DX_SPLITS": "1"}
+    old = {k: os.environ.get(k) for k in knobs}
+    os.environ.update(knobs)
+    try:
+        c = rt.Context(0)
+    finally:
+        for k, v in old.items():
+            os.environ.pop(k) if v is None else os.environ.update({k: v})
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("wtype", [O.Q4_0, O.Q8_0, O.Q4_K, O.Q6_K])
+@pytest.mark.parametrize("n,t", [(1500, 70), (1027, 300)])
+def test_dx_of_rows_of_wide_range(whole, wtype, n, t):
+    """Rows of dy with slices of 256 far below their largest, all summed by one workgroup: where the weight is
+    zero against the large values, the small ones' products are the result, to the same 2e-6.  Large values in the
+    first rows, the last, in between, next to zeros, everything tiny, and small slices alone.  (A range is shared by
+    256 rows, or 480 on 256-token tiles: those of the large values hold nothing else here.)"""
+    k = 512
+    w = O.Rng(1).vec_normal(n * k, 0.02).reshape(n, k)
+    big = np.array([5, 600, n - 1])
+    w[big, :64] = 0.0
+    blocks = O.quantize(wtype, w)
+    dense = O.dequantize(wtype, blocks, k).reshape(n, k).astype(np.float64)
+    assert (dense[big, :64] == 0).all()
+    dy = O.Rng(3).vec_normal(t * n, 1.0).reshape(t, n)
+    first, middle, last = slice(0, 480), slice(480, 960), slice(960, n)
+    dy[0::6, first] = 0.0
+    dy[0::6, big[0]] = 2.0 ** 45
+    dy[1::6, last] = 0.0
+    dy[1::6, big[2]] = -2.0 ** 50
+    dy[2::6, :960] = 0.0
+    dy[2::6, big[1]] = 2.0 ** 30
+    dy[3::6, first] = dy[3::6, last] = 0.0
+    dy[3::6, big[0]], dy[3::6, big[2]] = 2.0 ** 40, -2.0 ** 20
+    dy[4::6] *= 2.0 ** -100
+    dy[4::6, middle] = 0.0
+    dy[4::6, big[1]] = 2.0 ** -60
+    dy[5::6, middle] *= 2.0 ** -30
+    dx = np.zeros(t * k, np.float32)
+    rt.HipFrozen(wtype, blocks, n, k, ctx=whole).backward_input(dy, t, dx)
+    want = dy.astype(np.float64) @ dense
+    for cols in (slice(0, 64), slice(64, k)):
+        err = np.abs(dx.reshape(t, k) - want)[:, cols] / np.abs(want[:, cols]).max(axis=1, keepdims=True)
+        assert err.max() <= 2e-6, (cols, np.unravel_index(err.argmax(), err.shape), err.max())
