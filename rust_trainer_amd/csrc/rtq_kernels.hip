@@ -3619,6 +3619,7 @@ __device__ __forceinline__ void dx16_tile(const DxArgs& a) {
     if (pp == 0 && tl < a.T) {
       int ex = 0;
       (void)frexpf(mx, &ex);  // mx = f 2^ex, f in [0.5, 1): mx 2^(15 - ex) in [2^14, 2^15)
+      ex = max(ex, -111);     // 2^(15 - ex) stays a finite float
       const bool ok = mx > 0.0f && mx <= 3.0e38f;
       sSc[tl] = ok ? ldexpf(1.0f, 15 - ex) : 1.0f;
       sInv[tl] = (ok ? ldexpf(1.0f, ex - 15) : 1.0f) * a.wunsc;
@@ -3729,6 +3730,7 @@ __device__ __forceinline__ void dx32_tile(const DxArgs& a) {
       for (int k = 1; k < 8; k++) m = fmaxf(m, sRed[tid + k * 32]);
       int ex = 0;
       (void)frexpf(m, &ex);  // m = f 2^ex, f in [0.5, 1)
+      ex = max(ex, -111);    // 2^(15 - ex) stays a finite float
       const bool ok = m > 0.0f && m <= 3.0e38f;
       sRed[tid] = ok ? ldexpf(1.0f, 15 - ex) : 1.0f;
       sInv[tid] = (ok ? ldexpf(1.0f, ex - 15) : 1.0f) * a.wunsc;

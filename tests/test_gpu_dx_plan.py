@@ -104,3 +104,28 @@ def test_dx_of_rows_of_wide_range(whole, wtype, n, t):
     for cols in (slice(0, 64), slice(64, k)):
         err = np.abs(dx.reshape(t, k) - want)[:, cols] / np.abs(want[:, cols]).max(axis=1, keepdims=True)
         assert err.max() <= 2e-6, (cols, np.unravel_index(err.argmax(), err.shape), err.max())
+
+
+@pytest.fixture(scope="module", params=["0", "1"], ids=["default", "tok32"])
+def any_dx(request):
+    old = os.environ.get("RTQ_DX_32")
+    os.environ["RTQ_DX_32"] = request.param
+    try:
+        c = rt.Context(0)
+    finally:
+        os.environ.pop("RTQ_DX_32") if old is None else os.environ.update(RTQ_DX_32=old)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("t", [1, 8, 40])
+def test_dx_of_tiny_rows(any_dx, t):
+    """Rows whose largest value is below 2^-113, where 2^15 over it is no finite float."""
+    n, k = 600, 256
+    blocks = O.quantize(O.Q8_0, O.Rng(1).vec_normal(n * k, 0.02).reshape(n, k))
+    dy = O.Rng(3).vec_normal(t * n, 2.0 ** -118).reshape(t, n)
+    dx = np.zeros(t * k, np.float32)
+    rt.HipFrozen(O.Q8_0, blocks, n, k, ctx=any_dx).backward_input(dy, t, dx)
+    want = dy.astype(np.float64) @ O.dequantize(O.Q8_0, blocks, k).reshape(n, k).astype(np.float64)
+    # 2e-6 of the largest, and what 2^-126 at the range's bottom leaves: results near 2^-121 keep 2^-149 steps
+    assert (np.abs(dx.reshape(t, k) - want) <= 2e-6 * np.abs(want).max(axis=1, keepdims=True) + n * 2.0 ** -149).all()
