@@ -1619,7 +1619,7 @@ extern "C" __global__ __launch_bounds__(256) void rtq_mm32_q4_0(FwdArgs a) { mm_
 extern "C" __global__ __launch_bounds__(256) void rtq_mm32_q8_0(FwdArgs a) { mm_tile<FMT_Q8_0, 2, RTQ_MM32_RING>(a); }
 
 // ============================================================== forward GEMM, large grids (Q4_K / Q6_K)
-// rtq_mm_*'s ring kernel for the K-quants: 128 weight rows x 16 TTN tokens (TTN 4), four
+// rtq_mm_*'s ring kernel for the K-quants: 128 weight rows x 16 TTN tokens (TTN 4 or 2), four
 // waves of two row groups x all token tiles, the half-chunk operands - codes
 // (Q4_K in the Q4_0 layout, Q6_K in the Q8_0 layout), the sub-block scale words of the 128 rows,
 // the activation codes (Q8_K values as exact f16) - copied global -> LDS by buffer loads with an
@@ -1951,6 +1951,8 @@ __device__ __forceinline__ void mmk_tile(const FwdArgs& a) {
 
 extern "C" __global__ __launch_bounds__(256) void rtq_mmk64_q4_k(FwdArgs a) { mmk_tile<FMT_Q4_K, 4, RTQ_MM64_RING>(a); }
 extern "C" __global__ __launch_bounds__(256) void rtq_mmk64_q6_k(FwdArgs a) { mmk_tile<FMT_Q6_K, 4, RTQ_MM64_RING>(a); }
+extern "C" __global__ __launch_bounds__(256) void rtq_mmk32_q4_k(FwdArgs a) { mmk_tile<FMT_Q4_K, 2, RTQ_MM32_RING>(a); }
+extern "C" __global__ __launch_bounds__(256) void rtq_mmk32_q6_k(FwdArgs a) { mmk_tile<FMT_Q6_K, 2, RTQ_MM32_RING>(a); }
 
 // ============================================================== forward GEMM on int8 MFMA (Q4_0 / Q8_0)
 // rtq_mm64_*'s tiles (128 weight rows x 16 TTN tokens, TTN 4 here, four waves, the same RING-stage

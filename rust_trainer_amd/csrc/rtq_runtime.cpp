@@ -136,8 +136,10 @@ enum Kid {
   K_MM32_Q8_0,
   K_MMI8_64_Q4_0,  // the 128 x 64 tiles with the block sums on int8 MFMA
   K_MMI8_64_Q8_0,
-  K_MMK64_Q4_K,    // the LDS-ring kernel for the K-quants: 128 x 64 tiles
+  K_MMK64_Q4_K,    // the LDS-ring kernel for the K-quants: 128 x 64 and 128 x 32 tiles
   K_MMK64_Q6_K,
+  K_MMK32_Q4_K,
+  K_MMK32_Q6_K,
   K_BWD_PREP,
   K_DX,          // + format
   K_DX16 = K_DX + F_COUNT,  // + format: t <= 16
@@ -181,7 +183,7 @@ constexpr const char* kKernelNames[] = {
     "rtq_mm_q4_0",          "rtq_mm_q8_0",
     "rtq_mm64_q4_0",        "rtq_mm64_q8_0",        "rtq_mm32_q4_0",        "rtq_mm32_q8_0",
     "rtq_mmi8_64_q4_0",     "rtq_mmi8_64_q8_0",
-    "rtq_mmk64_q4_k",       "rtq_mmk64_q6_k",
+    "rtq_mmk64_q4_k",       "rtq_mmk64_q6_k",       "rtq_mmk32_q4_k",       "rtq_mmk32_q6_k",
     "rtq_bwd_prep",
     "rtq_dx_q4_0",          "rtq_dx_q8_0",          "rtq_dx_q4_k",          "rtq_dx_q6_k",
     "rtq_dx16_q4_0",        "rtq_dx16_q8_0",        "rtq_dx16_q4_k",        "rtq_dx16_q6_k",
@@ -240,8 +242,8 @@ struct rtq_ctx {
   int g64_min = -1;   // fewest 64-token g-partial workgroups (else 16-token ones): -1 = CUs / 2 (RTQ_G64_MIN)
   int fwd_mm = -1;    // large-grid forward: -1 automatic, 0 never, 1 / 2 / 3 the 128- / 64- / 32-token tiles
                       // whenever the format allows (RTQ_FWD_MM)
-  int fwd_mmk = -1;   // K-quant ring forward (rtq_mmk64_*; RTQ_FWD_MMK): -1 automatic, 0 never, else whenever
-                      // the shape allows
+  int fwd_mmk = -1;   // K-quant ring forward (rtq_mmk*_*; RTQ_FWD_MMK): -1 automatic, 0 never, 1 / 2 the 64- /
+                      // 32-token tiles whenever the shape allows
   int dxv = 1;        // t == 1 dx on f32 FMAs (rtq_dxv1_*; RTQ_DXV=0: rtq_dx16_*)
   int dxv_wpc = 3;    // rtq_dxv1_* row splits for about this many workgroups per CU (RTQ_DXV_WPC)
   int gemvq = 1;      // one-launch GEMV for t <= 4 (rtq_gemvq*_*; RTQ_GEMVQ=0: activation kernel + GEMM)
@@ -667,6 +669,20 @@ rtq_status enqueue_backward_dense(rtq_ctx* c, const rtq_weight* w, const float* 
   return RTQ_OK;
 }
 
+// Whether a Q4_0 / Q8_0 forward is faster on 32-token tiles (mm32 of them) than on the eight-wave tiles (`tiles`
+// of wrg row groups of 16), both of one whole call in us: a launch and its start, then per 1024 columns what a
+// tile takes beside the others on its CU (32-token) or per round of the chip (eight-wave).  Over 1714 calls of 512
+// to 65536 rows, 256 to 9728 columns and 17 to 1000 tokens (profiles/forward_small_grids.md) the choice is the
+// slower one by more than 5% in 7, by 14% at most.  A lower limit of 1.5 tiles per CU took the slower one in a
+// seventh of them, by up to 2.2 times: 8192 x 1024 at 140 tokens 26 us against 17, 40000 x 1024 at 25 33 / 22
+bool fwd_mm32_wins(const rtq_ctx* c, const rtq_weight* w, int64_t mm32, int wrg, int64_t tiles) {
+  static const double beside[4] = {8.0, 10.3, 13.1, 18.0}, start[3] = {2.0, 2.8, 4.2}, round[3] = {2.3, 2.6, 3.2};
+  const double k = w->cols / 1024.0;
+  const double one = w->type == RTQ_TYPE_Q4_0 ? 8.4 : beside[0];  // alone on its CU
+  const int64_t n = std::min<int64_t>(std::max<int64_t>(cdiv(mm32, c->cu_count), 1), 4);
+  return 6.0 + k * (n == 1 ? one : beside[n - 1]) < 5.0 + cdiv(tiles, c->cu_count) * (start[wrg - 1] + k * round[wrg - 1]);
+}
+
 // ------------------------------------------------------------------ enqueue: forward
 // y = x.W^T (+bias) (+ s h.B^T);  isums (debug) receives the per-block integer sums.
 // hp_keep (optional, nhp * t * r floats): the LoRA-down partials go there instead of the workspace,
@@ -793,12 +809,17 @@ rtq_status enqueue_forward(rtq_ctx* c, const rtq_weight* w, const float* x, int6
   const int64_t rg_per_wg = p.skinny ? kFwdSkinnyRG : (w8 ? wrg : wide_rg(w->type));
   const int64_t gx = cdiv(w->Np / 16, rg_per_wg);
   // the large-grid kernels (tiles of 128 rows x 128, 64 or 32 tokens; tokens < t only).  Automatic:
-  //  * the int8-MFMA form on 64-token tiles where those give 1.6 workgroups per CU (Q4_0: the f16 form on
-  //    128-token tiles from 16 of those per CU, and on rows of 256 columns from one); both forms agree bit for
-  //    bit without an adapter;
-  //  * else 32-token tiles where they give 1.5 workgroups per CU (below, the eight-wave tiles, which split
-  //    the columns over their waves, are as fast on long rows);
-  //  * else the eight-wave tiles.
+  //  * the int8-MFMA form on 64-token tiles where those give 1.6 workgroups per CU (on a row count that is no
+  //    multiple of 4 where the 128-token tiles give one: Q8_0 30710 x 640, 105 tokens, 32-token tiles 23 us, int8
+  //    25); both forms agree bit for bit without an adapter.  Q4_0: the f16 form on 128-token tiles
+  //    - from 16 of those per CU;
+  //    - where they need one round of the chip (two a CU) and the int8 ones, three a CU, a second: 8192 x 1024 at
+  //      1024 tokens 39 / 40 us, 28672 x 1024 at 256 35 / 37, 14336 x 256 at 512 18 / 20;
+  //    - past 64 tokens on a row count that is no multiple of 4, whose stores cost the int8 form more, up to 1024
+  //      columns: 53565 rows, 384 tokens, 256, 1024 columns 62 / 77, 99 / 108 (at 2048 154 / 158, but 121 / 115 at
+  //      256 tokens);
+  //    - on rows of 256 columns from one per CU, where the int8 form is up to 16% faster or 27% slower;
+  //  * else 32-token or eight-wave tiles, by the time of each (fwd_mm32_wins).
   // Measured per forward kernel, us, i8-64 / f16-128 / f16-32 / eight-wave: Q4_0 4096 x 1024 at 256, 512, 1001,
   // 2048 tokens 17 / 23 / 13 / 18, 18 / 24 / 16 / 26, 22 / 26 / 28 / 49, 38 / 36 / 46 / 89; 6144 x 1024 at
   // 1001, 2048 28 / 34 / 36 / 66, 50 / 53 / 66 / 129; 151936 x 1024 at 37, 256, 512 69 / 71 / 91 / 103,
@@ -816,22 +837,37 @@ rtq_status enqueue_forward(rtq_ctx* c, const rtq_weight* w, const float* x, int6
     else if (c->fwd_mm == 2) mm_ttn = 4;
     else if (c->fwd_mm == 3) mm_ttn = 2;
     else if (c->fwd_mm < 0) {
-      const bool q4_f16 = w->type == RTQ_TYPE_Q4_0 && (mm128 >= 16 * cu || (w->cols <= 256 && mm128 >= cu));
-      if (5 * mm64 >= 8 * cu) mm_ttn = q4_f16 ? 8 : 4;
-      else if (2 * mm32 >= 3 * cu) mm_ttn = 2;
+      const bool q4_f16 = w->type == RTQ_TYPE_Q4_0 &&
+                          (mm128 >= 16 * cu || (mm64 > 3 * cu && mm64 <= 4 * cu && mm128 <= 2 * cu) ||
+                           (mm128 >= cu && (w->cols <= 256 || (w->cols <= 1024 && w->rows % 4 && t > 64))));
+      if (5 * mm64 >= 8 * cu && (w->rows % 4 == 0 || mm128 >= cu)) mm_ttn = q4_f16 ? 8 : 4;
+      else if (fwd_mm32_wins(c, w, mm32, wrg, gx * gy)) mm_ttn = 2;
     }
     // a Q4_0 weight's 64-token tiles asked for by RTQ_FWD_MM stay the f16 kernel's
     mmi8 = mm_ttn >= 4 && (c->fwd_i8 == 1 || (c->fwd_i8 < 0 && (w->type == RTQ_TYPE_Q8_0 || (c->fwd_mm < 0 && mm_ttn == 4))));
     if (mmi8) mm_ttn = 4;
   }
   const bool mm = mm_ttn > 0;
-  // K-quants: the LDS-ring kernel where its 128 x 64 tiles (of tokens < t) give half the CUs two workgroups,
-  // else the tile kernel (rtq_fwd_*_w).  Measured per forward kernel, ring / tile, us (and workgroups):
-  // Q4_K 9728 x 2560 at 200, 400, 1001 tokens 49 / 42 (304), 64 / 70 (532), 108 / 147 (1216); Q6_K 2560 x
-  // 9728 at 1001, 2048 183 / 143 (320), 291 / 306 (640); Q4_K 2560 x 4096 at 1001, 2048 74 / 61 (320),
-  // 101 / 115 (640); Q4_K 14336 x 4096 at 100, 200 58 / 48 (224), 77 / 81 (448)
-  const int64_t mmk_tiles = mm_rows * cdiv(t, 64);
-  const bool mmk = !p.skinny && !isums && kq && (c->fwd_mmk > 0 || (c->fwd_mmk < 0 && 2 * mmk_tiles >= 3 * c->cu_count));
+  // K-quants: the LDS-ring kernel from a number of its 128 x 64 tiles (of tokens < t) per CU, else the tile kernel
+  // (rtq_fwd_*_w), whose waves split the columns: 0.75 per CU at up to 512 columns, rising to 1.5 (Q4_K; reached at
+  // 1102 columns) or 1.75 (Q6_K; 1299).  Measured per call, ring / tile, over 512 to 120000 rows and 17 to 1024
+  // tokens (profiles/forward_small_grids.md), by tiles per CU: 256 columns 0.5 1.05, 0.75 0.77, 1 0.72 - 0.91, 1.5
+  // 0.67; 512: 0.5 1.1 - 1.18, 0.75 0.93, 1 0.8; 1024, Q4_K: 1 1.02, 1.25 1.06, 1.5 0.95, 2 0.8; Q6_K: 1.25 1.14,
+  // 1.5 1.01, 2 0.86; from 2048, Q4_K: 1.25 1.13 - 1.26, 1.5 1.01 - 1.08, 1.75 0.95; Q6_K: 1.5 1.08 - 1.21, 1.75
+  // 0.96 - 1.08, 2 0.84 - 0.96.  (One limit of 1.5 had 14148 x 256 at 79 tokens on 14.9 us instead of 10.8.)
+  // Its 32-token tiles up to 32 tokens (0.83 - 0.95 of the 64-token ones' time; of the tile kernel's from one per
+  // CU 0.9 - 1.05), and at up to 512 columns above half a 64-token one per CU (0.7 - 1.01 of the tile kernel's)
+  const int64_t mmk_tiles = mm64;
+  const double mmk_min = std::min(w->type == RTQ_TYPE_Q4_K ? 1.5 : 1.75, 0.75 + 0.65 * (std::max<int64_t>(w->cols, 512) / 512.0 - 1.0));
+  int mmk_ttn = 0;  // token tiles of 16 per workgroup of the chosen ring kernel, 0: none
+  if (!p.skinny && !isums && kq) {
+    if (c->fwd_mmk > 0) mmk_ttn = c->fwd_mmk == 2 ? 2 : 4;
+    else if (c->fwd_mmk < 0) {
+      if (t <= 32) mmk_ttn = mmk_tiles >= std::min(mmk_min, 1.0) * c->cu_count ? 2 : 0;
+      else if (mmk_tiles >= mmk_min * c->cu_count) mmk_ttn = 4;
+      else if (w->cols <= 512 && 2 * mmk_tiles > c->cu_count) mmk_ttn = 2;
+    }
+  }
   const int64_t mm_tiles = mm_ttn == 8 ? mm128 : mm_ttn == 4 ? mm64 : mm32;
   // split K across workgroups when the output alone gives too few of them (atomics into a
   // zeroed y); every split keeps at least one half chunk per wave (K-quants: one super-block of
@@ -841,7 +877,7 @@ rtq_status enqueue_forward(rtq_ctx* c, const rtq_weight* w, const float* x, int6
   // get the same bits
   const int64_t tiles = gx * gy;
   int64_t ks = 1;
-  if (!isums && !mm && !mmk && !w8 && tiles < c->cu_count) {
+  if (!isums && !mm && !mmk_ttn && !w8 && tiles < c->cu_count) {
     const int64_t want = cdiv(p.skinny ? 2 * c->cu_count : c->cu_count, tiles);
     ks = std::max<int64_t>(1, std::min<int64_t>(want, Kc / (kq ? 8 : 2)));
   }
@@ -849,7 +885,7 @@ rtq_status enqueue_forward(rtq_ctx* c, const rtq_weight* w, const float* x, int6
   if (kq) kcps = roundup(kcps, 2);
   ks = cdiv(Kc, kcps);
 
-  const bool xbs = mmk && w->type == RTQ_TYPE_Q4_K;  // code sums instead of the replicated scales
+  const bool xbs = mmk_ttn && w->type == RTQ_TYPE_Q4_K;  // code sums instead of the replicated scales
   uint16_t* xdh = mm || xbs ? ar.take<uint16_t>(p.xdh_bytes / 2) : nullptr;
   if (ar.off > ar.cap) return fail(RTQ_ERR_INVALID, "internal: workspace too small");
   ActArgs aa{x, (int)t, (int)w->cols, (int)p.Tp, (int)w->Kp, xq, xd, nullptr, 0.0f, lora ? la : nullptr, (int)r, hp,
@@ -892,11 +928,12 @@ rtq_status enqueue_forward(rtq_ctx* c, const rtq_weight* w, const float* x, int6
   if (mmi8)
     return launch(c, K_MMI8_64_Q4_0 + (w->type == RTQ_TYPE_Q4_0 ? 0 : 1), dim3((unsigned)mm_tiles), dim3(256), st, fa,
                   mmi8_lds_bytes(w->type, 4, RTQ_MM64_RING));
-  if (mmk) {
+  if (mmk_ttn) {
     if (!fa.wq || !fa.wd || !fa.wsb || !fa.xq || !fa.xd || !fa.y || (xbs && !fa.xdh))
       return fail(RTQ_ERR_INVALID, "internal: rtq_mmk_* operand missing");
-    return launch(c, K_MMK64_Q4_K + (w->type == RTQ_TYPE_Q4_K ? 0 : 1), dim3((unsigned)mmk_tiles), dim3(256), st, fa,
-                  mmk_lds_bytes(w->type, 4, RTQ_MM64_RING));
+    return launch(c, (mmk_ttn == 4 ? K_MMK64_Q4_K : K_MMK32_Q4_K) + (w->type == RTQ_TYPE_Q4_K ? 0 : 1),
+                  dim3((unsigned)(mmk_ttn == 4 ? mmk_tiles : mm32)), dim3(256), st, fa,
+                  mmk_lds_bytes(w->type, mmk_ttn, mmk_ttn == 4 ? RTQ_MM64_RING : RTQ_MM32_RING));
   }
   if (mm) {
     const int ring = mm_ttn == 8 ? RTQ_MM_RING : mm_ttn == 4 ? RTQ_MM64_RING : RTQ_MM32_RING;
