@@ -997,7 +997,7 @@ DxPlan dx_plan(const rtq_ctx* c, const rtq_weight* w, int64_t t) {
       const bool wide = kind == 1;
       if (c->dx_wide >= 0 ? wide != (c->dx_wide == 1) : wide && c->dx_32 > 0) continue;
       const int64_t tiles = Kc * cdiv(t, wide ? 256 : 64);
-      for (int64_t sp = 1; sp <= (wide ? 32 : 16) && (sp == 1 || cdiv(steps, sp) >= 4); sp++) {
+      for (int64_t sp = 1; sp <= (wide ? 32 : 16) && (sp == 1 || cdiv(steps, sp) >= (wide ? 4 : 1)); sp++) {
         int64_t nf;
         const double us = dx_cost(c, wide, kq, steps, tiles, sp, &nf);
         if (us < best) {
