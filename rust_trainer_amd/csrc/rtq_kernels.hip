@@ -618,7 +618,7 @@ __device__ __forceinline__ void act_prep(const ActArgs& a) {
         }
         sx[tile_unit(w + 4 * i, lane)] = x4;
       }
-    } else {
+    } else if (a.A) {  // uniform
       f4 xv[4];
 #pragma unroll
       for (int i = 0; i < 4; i++) {
@@ -629,12 +629,23 @@ __device__ __forceinline__ void act_prep(const ActArgs& a) {
 #pragma unroll
       for (int i = 0; i < 4; i++) sx[tile_unit(w + 4 * i, lane)] = xv[i];
     }
-    __syncthreads();
+    // (K % 32 == 0: a thread's 16 columns are all in or all out)
+    if (NORM || a.A || a.sg) {  // uniform
+      __syncthreads();
 #pragma unroll
-    for (int i = 0; i < 4; i++) {  // K % 32 == 0: a thread's 16 columns are all in or all out
-      const f4 x4 = sx[tile_unit(tl, 4 * sg + i)];
+      for (int i = 0; i < 4; i++) {
+        const f4 x4 = sx[tile_unit(tl, 4 * sg + i)];
 #pragma unroll
-      for (int e = 0; e < 4; e++) v[4 * i + e] = x4[e];
+        for (int e = 0; e < 4; e++) v[4 * i + e] = x4[e];
+      }
+    } else {  // no adapter: straight to the thread, no barrier (0.2 - 0.4 us of a small forward)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const f4 x4 = t < a.T && kk < a.K ? *reinterpret_cast<const f4*>(a.x + (int64_t)t * a.K + kk + 4 * i)
+                                          : f4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[4 * i + e] = x4[e];
+      }
     }
     _Float16 q[16];  // codes: exact small integers
     float dstore;    // the block scale as the dot products use it
