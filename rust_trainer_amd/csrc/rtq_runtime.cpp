@@ -983,6 +983,11 @@ double dx_cost(const rtq_ctx* c, bool wide, bool kq, int64_t steps, int64_t tile
   if (last) us += len * (last > cu ? both : alone) + start;
   return us + (double)((splits - 1) * (tiles - *nfull)) * (wide ? 0.05 : 0.02);
 }
+// The most 64-token partial tiles that a t > 16 plan adds: no plan of the model alone over 2 to 120 K chunks, 10240
+// tokens and 5000 steps has more, so that it binds none and rtq_ctx_reserve has a bound that grows with the weight
+int64_t dx_part_cap(const rtq_ctx* c, int64_t steps) {
+  return std::min<int64_t>(640 + 12 * steps, 4608 + 3 * steps) * c->cu_count / 256;
+}
 DxPlan dx_plan(const rtq_ctx* c, const rtq_weight* w, int64_t t) {
   DxPlan p;
   p.tok16 = t <= 16;
@@ -1000,7 +1005,7 @@ DxPlan dx_plan(const rtq_ctx* c, const rtq_weight* w, int64_t t) {
       for (int64_t sp = 1; sp <= (wide ? 32 : 16) && (sp == 1 || cdiv(steps, sp) >= (wide ? 4 : 1)); sp++) {
         int64_t nf;
         const double us = dx_cost(c, wide, kq, steps, tiles, sp, &nf);
-        if (us < best) {
+        if (us < best && (sp - 1) * (tiles - nf) * (wide ? 4 : 1) <= dx_part_cap(c, steps)) {
           best = us;
           p.wide = wide;
           p.nfull = nf;
@@ -1046,12 +1051,36 @@ size_t bwd_ws_bytes(const rtq_ctx* c, const rtq_weight* w, int64_t t, int64_t r)
   const int64_t sl = lora_slices(n) + lora_slices(k);
   if (is_dense(w->type)) {
     const size_t hg = (size_t)((2 + (dense_fast(w, t) ? sl : 0)) * t * std::max<int64_t>(r, 0)) * 4;
-    return hg + (dense_fast(w, t) ? (size_t)(dense_bwd_plan(c, w, std::max<int64_t>(t, 1)).nsplit * t * k) * 4 : 0) + 6 * 256;
+    const int64_t ns = dense_fast(w, t) ? dense_bwd_plan(c, w, std::max<int64_t>(t, 1)).nsplit : 1;
+    return hg + (ns > 1 ? (size_t)(ns * t * k) * 4 : 0) + 6 * 256;  // one split: dx itself
   }
   return (size_t)((2 + sl) * t * std::max<int64_t>(r, 0)) * 4 + dx_plan(c, w, std::max<int64_t>(t, 1)).part_floats * 4 +
          (size_t)(lora_slices(n) * t) * 4 + 7 * 256;
 }
 
+// at least bwd_ws_bytes of every weight of at most w's rows and columns at every number of tokens up to t and
+// ranks up to r (the plans are not monotonic: fewer tokens or columns can split more)
+size_t bwd_ws_bound(const rtq_ctx* c, const rtq_weight* w, int64_t t, int64_t r) {
+  const int64_t n = w->rows, k = w->cols, Kc = w->Kp / 128, steps = w->Np / 32, cu = c->cu_count, t16 = std::min<int64_t>(t, 16);
+  const int64_t tg = cdiv(t, 64), tiles = tg * Kc, tiles4 = cdiv(t, 256) * 4 * Kc;
+  // splits times columns: at most the most splits, and S / chunks, rounded up
+  auto rows16 = [&](int64_t most, int64_t S) { return std::min(std::max<int64_t>(most, 1) * Kc, S + Kc) * 128; };
+  int64_t part = rows16(std::min<int64_t>(cdiv(steps, 4), 256), 2 * cu) * t16;
+  part = std::max(part, rows16(cdiv(w->Np, 128), c->dxv_wpc * cu));
+  if (t > 16) {
+    int64_t more = std::min(dx_part_cap(c, steps), std::max(15 * tiles, 31 * tiles4));
+    if (c->dx_32 > 0) more = 15 * tiles;
+    part = std::max(part, (tiles + more) * 8192);
+  }
+  if (c->dx_splits > 0) {
+    const int64_t sp = std::min<int64_t>(c->dx_splits, 256);
+    part = std::max({part, sp * Kc * 128 * t16, (tiles + (std::min<int64_t>(sp, 64) - 1) * tiles4) * 8192});
+  }
+  // trainer-native: more than one split only on 32-token tiles, fewer than 2 cu of them
+  part = std::max(part, std::min(4 * cu * 2048, std::max<int64_t>(steps / 8, 1) * t * k));
+  const int64_t sl = lora_slices(n) + lora_slices(k);
+  return (size_t)((2 + sl) * t * std::max<int64_t>(r, 0)) * 4 + (size_t)part * 4 + (size_t)(lora_slices(n) * t) * 4 + 7 * 256;
+}
 
 // dx (+)= dy.W (accumulate: FrozenMatmul::backward_input; otherwise dx is overwritten, as
 // Linear::backward returns a fresh dx); with LoRA also dx += g.A, ga += g^T x, gb += (s dy)^T h
@@ -1401,22 +1430,13 @@ rtq_status rtq_ctx_reserve(rtq_ctx* c, int64_t max_t, int64_t max_rows, int64_t 
   fake.Np = roundup(max_rows, RTQ_ROW_PAD);
   fake.Kp = roundup(max_cols, RTQ_CHUNK_Q);
   fake.type = RTQ_TYPE_Q4_0;
-  size_t need = fwd_ws_bytes(fwd_plan(&fake, max_t, max_rank));
-  // the dx plans' split tiles: fewer tokens or a narrower weight can need more of them
-  const int64_t step = std::max<int64_t>(64, roundup(cdiv(max_t, 1024), 64));
-  for (int type : {RTQ_TYPE_Q4_0, RTQ_TYPE_Q4_K}) {
+  size_t need = bwd_ws_bound(c, &fake, max_t, max_rank);
+  for (int type : {RTQ_TYPE_Q4_0, RTQ_TYPE_F32}) {
     fake.type = type;
-    for (int64_t k = max_cols; k > 0; k -= 512) {
-      fake.cols = k;
-      fake.Kp = roundup(k, RTQ_CHUNK_Q);
-      for (int64_t t = 64; t < max_t; t += step) need = std::max(need, bwd_ws_bytes(c, &fake, t, max_rank));
-      for (int64_t t : {std::min<int64_t>(max_t, 16), max_t}) need = std::max(need, bwd_ws_bytes(c, &fake, t, max_rank));
-    }
+    for (int64_t t : {std::min<int64_t>(max_t, 16), max_t})
+      for (int64_t r : {std::min<int64_t>(max_rank, RTQ_LDS_RANK), max_rank})
+        need = std::max(need, fwd_ws_bytes(fwd_plan(&fake, t, r)));
   }
-  fake.cols = max_cols;
-  fake.Kp = roundup(max_cols, RTQ_CHUNK_Q);
-  fake.type = RTQ_TYPE_F32;
-  need = std::max({need, fwd_ws_bytes(fwd_plan(&fake, max_t, max_rank)), bwd_ws_bytes(c, &fake, max_t, max_rank)});
   RTQ_TRY(ensure_ws(c, need));
   return RTQ_OK;
 }
