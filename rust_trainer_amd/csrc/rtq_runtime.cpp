@@ -246,6 +246,7 @@ struct rtq_ctx {
                       // 32-token tiles whenever the shape allows
   int dxv = 1;        // t == 1 dx on f32 FMAs (rtq_dxv1_*; RTQ_DXV=0: rtq_dx16_*)
   int dxv_wpc = 3;    // rtq_dxv1_* row splits for about this many workgroups per CU (RTQ_DXV_WPC)
+  int dense_split = 1;  // trainer-native products on split bf16 MFMAs where they fit (RTQ_DENSE_SPLIT=0: never)
   int gemvq = 1;      // one-launch GEMV for t <= 4 (rtq_gemvq*_*; RTQ_GEMVQ=0: activation kernel + GEMM)
   int gemvq_wpc = 0;  // its waves per CU (RTQ_GEMVQ_WPC; 0: automatic)
   int fwd_i8 = -1;    // int8-MFMA forwards (rtq_mmi8_*; RTQ_FWD_I8): -1 automatic (Q8_0 weights), 0 never,
@@ -447,7 +448,9 @@ int64_t lora_slices(int64_t n) { return roundup(cdiv(std::max<int64_t>(n, 1), RT
 // 90; 4096 x 4096 forward 203 / 53, 326 / 105, 518 / 225, backward 339 / 27, 550 / 155, 792 / 325
 bool dense_fast(const rtq_weight* w, int64_t t) {
   const uint64_t lim = 1ull << 31, N = (uint64_t)w->rows, K = (uint64_t)w->cols;
-  return K % 32 == 0 && (uint64_t)t * N * 4 < lim && (uint64_t)t * K * 4 < lim && N * K * 4 < lim;
+  if (w->ctx && !w->ctx->dense_split) return false;
+  return K % 32 == 0 && (uint64_t)t * N * 4 < lim && (uint64_t)t * K * 4 < lim && N * K * 4 < lim &&
+         lora_slices(w->rows) + lora_slices(w->cols) <= 65535;  // rtq_bwd_prep's grid
 }
 // forward workspace of the strided GEMM: h
 size_t dense_min_bytes(int64_t t, int64_t r) { return (size_t)(t * std::max<int64_t>(r, 0)) * 4 + 2 * 256; }
@@ -1369,6 +1372,7 @@ rtq_status rtq_ctx_create(int device, rtq_ctx** out) {
   if (const char* e = getenv("RTQ_FWD_MM")) c->fwd_mm = std::min(std::max(atoi(e), 0), 3);
   if (const char* e = getenv("RTQ_FWD_I8")) c->fwd_i8 = std::min(std::max(atoi(e), -1), 1);
   if (const char* e = getenv("RTQ_FWD_MMK")) c->fwd_mmk = std::min(std::max(atoi(e), -1), 2);
+  if (const char* e = getenv("RTQ_DENSE_SPLIT")) c->dense_split = atoi(e) ? 1 : 0;
   if (const char* e = getenv("RTQ_GEMVQ")) c->gemvq = atoi(e) ? 1 : 0;
   if (const char* e = getenv("RTQ_DXV")) c->dxv = atoi(e) ? 1 : 0;
   if (const char* e = getenv("RTQ_DXV_WPC")) c->dxv_wpc = std::max(1, std::min(16, atoi(e)));

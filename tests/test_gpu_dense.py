@@ -1,9 +1,12 @@
 """The split-bf16 products of the trainer-native weights (rtq_dense_*) against float64, at the edges of
 their tiles: one token, 31 / 32 / 33 and 64 / 65 tokens, rows that leave a tile or a 32-row step ragged,
 a row count that is no multiple of 4 (scalar dy loads), one 32-column block, enough tiles for the
-64-token form, several row splits.  An f32 dot of n terms is within (n / 2 + 2) 2^-24 of the sum of its
+64-token form either way, several row splits; each test asserts which kernels ran.  The strided f32 GEMM, which
+takes the calls that do not fit these kernels, runs through the same cases (RTQ_DENSE_SPLIT=0).  An f32 dot of n terms is within (n / 2 + 2) 2^-24 of the sum of its
 terms' magnitudes however it is ordered; the products here leave out terms below 2^-30 each, so the
 bound below is (n / 16 + 4) 2^-24 of that sum (a rounding per 32-element step and of the split's parts)."""
+import os
+
 import numpy as np
 import pytest
 
@@ -13,7 +16,7 @@ import rust_trainer_amd as rt
 pytestmark = pytest.mark.gpu
 
 SHAPES = [(64, 32, 1), (37, 96, 31), (65, 64, 32), (200, 160, 33), (130, 256, 64), (257, 128, 65), (1030, 2048, 17),
-          (4096, 1024, 600)]
+          (4096, 1024, 600), (70, 4096, 520), (1030, 8192, 257)]
 
 
 def _weight(ctx, kind, n, k):
@@ -33,9 +36,32 @@ def ctx():
     c.close()
 
 
+@pytest.fixture(scope="module", params=["split", "gemm"])
+def either(request, ctx):
+    if request.param == "split":
+        yield "split", ctx
+        return
+    old = os.environ.get("RTQ_DENSE_SPLIT")
+    os.environ["RTQ_DENSE_SPLIT"] = "0"
+    try:
+        c = rt.Context(0)
+    finally:
+        os.environ.pop("RTQ_DENSE_SPLIT") if old is None else os.environ.update(RTQ_DENSE_SPLIT=old)
+    yield "gemm", c
+    c.close()
+
+
+def _kernels(kind, n, k, t):
+    """The product kernels of a forward and a backward on 256 CUs."""
+    tok = [64 if -(-out // 64) * -(-t // 64) >= 512 else 32 for out in (n, k)]
+    q8 = "_q8" if kind == "tq8" else ""
+    return {f"rtq_dense_fwd{tok[0]}{q8}", f"rtq_dense_bwd{tok[1]}{q8}"}
+
+
 @pytest.mark.parametrize("kind", ["f32", "tq8"])
 @pytest.mark.parametrize("n,k,t", SHAPES)
-def test_dense_products(ctx, kind, n, k, t):
+def test_dense_products(either, kind, n, k, t):
+    path, ctx = either
     hw, w = _weight(ctx, kind, n, k)
     x = O.Rng(2).vec_normal(t * k, 1.0).reshape(t, k)
     dy = O.Rng(3).vec_normal(t * n, 1.0).reshape(t, n) * np.exp(O.Rng(4).vec_normal(t, 2.0))[:, None].astype(np.float32)
@@ -47,8 +73,11 @@ def test_dense_products(ctx, kind, n, k, t):
     x64, dy64, a64, b64 = (v.astype(np.float64) for v in (x, dy, a, b))
 
     def close(got, want, size, terms):
-        assert (np.abs(np.asarray(got, np.float64).reshape(want.shape) - want) <= (terms / 16 + 4) * eps * size).all()
+        bound = terms / 16 + 4 if path == "split" else terms / 2 + 2
+        assert (np.abs(np.asarray(got, np.float64).reshape(want.shape) - want) <= bound * eps * size).all()
 
+    ctx.set_timing(True)
+    ctx.reset_timing()
     y = lin.forward(x, t)
     h = x64 @ a64.T
     size = np.abs(x64) @ np.abs(w.T) + np.abs(lin.bias) + 2 * (np.abs(x64) @ np.abs(a64.T)) @ np.abs(b64.T)
@@ -63,6 +92,12 @@ def test_dense_products(ctx, kind, n, k, t):
     dx = dx0.copy()
     hw.backward_input(dy, t, dx)  # accumulates
     close(dx, dy64 @ w + dx0.reshape(t, k), np.abs(dy64) @ np.abs(w) + np.abs(dx0.reshape(t, k)), n)
+    ran = {name for name in ctx.timing() if "dense" in name or "gemm" in name}
+    ctx.set_timing(False)
+    if path == "split":
+        assert ran == _kernels(kind, n, k, t), ran
+    else:
+        assert ran and all(name.startswith("rtq_m_gemm") for name in ran - {"rtq_dense_bias"}), ran
 
 
 @pytest.mark.parametrize("kind", ["f32", "tq8"])

@@ -118,6 +118,17 @@ def any_dx(request):
     c.close()
 
 
+@pytest.mark.parametrize("wtype,n,k,t", [(O.Q6_K, 426, 256, 22), (O.Q4_0, 70, 96, 17), (O.Q8_0, 300, 544, 70)])
+def test_dx_of_small_weights(any_dx, wtype, n, k, t):
+    """Weights of a few 32-row steps, split down to one step a workgroup by the default plan."""
+    blocks = O.quantize(wtype, O.Rng(1).vec_normal(n * k, 0.02).reshape(n, k))
+    dy = O.Rng(3).vec_normal(t * n, 1.0).reshape(t, n)
+    dx = np.zeros(t * k, np.float32)
+    rt.HipFrozen(wtype, blocks, n, k, ctx=any_dx).backward_input(dy, t, dx)
+    want = dy.astype(np.float64) @ O.dequantize(wtype, blocks, k).reshape(n, k).astype(np.float64)
+    assert (np.abs(dx.reshape(t, k) - want) <= 2e-6 * np.abs(want).max(axis=1, keepdims=True)).all()
+
+
 @pytest.mark.parametrize("t", [1, 8, 40])
 def test_dx_of_tiny_rows(any_dx, t):
     """Rows whose largest value is below 2^-113, where 2^15 over it is no finite float."""

@@ -524,6 +524,7 @@ def ctx_mmk(request):
     """A context that sends every wide K-quant forward through the LDS-ring kernel's 64-token
     (RTQ_FWD_MMK=1) or 32-token (2) tiles"""
     c = _context({"RTQ_FWD_MMK": request.param})
+    c.ring = "rtq_mmk64" if request.param == "1" else "rtq_mmk32"
     yield c
     c.close()
 
@@ -548,7 +549,7 @@ def test_linear_forward_kquant_ring_matches_oracle(ctx_mmk, wtype, n, k, t, r):
     y = lin.forward(x, t)
     ran = ctx_mmk.timing()
     ctx_mmk.set_timing(False)
-    assert any(name.startswith("rtq_mmk") for name in ran), ran
+    assert any(name.startswith(ctx_mmk.ring) for name in ran), ran
     want = O.linear_forward(wtype, blocks, n, k, x, bias=bias, nthreads=8, **kw)
     assert rel_err(y, want) <= TOL
 

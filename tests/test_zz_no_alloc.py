@@ -7,7 +7,8 @@ library's file-scope device array) against rtq_linear_forward_d on the same inpu
   every output equals the allocating entry point's within 1e-5 (the kernels are the same);
 * the device's free memory does not move across the no-allocation calls;
 * a forward whose workspace exceeds the array is refused before any launch, naming the maximum;
-* trainer-native (F32, TQ8_0) weights allocate nothing either and give the allocating path's output.
+* trainer-native (F32, TQ8_0) weights allocate nothing either and give the allocating path's output, also where
+  the adapter's slice partials exceed the array and the call runs on the strided f32 GEMM.
 """
 import ctypes
 
@@ -91,8 +92,7 @@ def test_noalloc_forward_refuses_what_it_cannot_serve():
     assert rc == 1 and b"maximum" in _ffi.lib().rtq_last_error()
     torch.cuda.synchronize()
     assert bool((y == 5.0).all()), "a refused call wrote its output"
-    # trainer-native weights run on the f32 GEMM and allocate nothing either: same output as the
-    # allocating entry point
+    # trainer-native weights allocate nothing either: same output as the allocating entry point
     stream = torch.cuda.current_stream().cuda_stream
     for wf in (rt.HipFrozen.f32(O.Rng(5).vec_normal(96 * 256, 0.02), 96, 256, ctx=ctx),
                rt.HipFrozen.q8_0(O.Rng(6).vec_normal(96 * 256, 0.02), 96, 256, ctx=ctx)):
@@ -109,3 +109,47 @@ def test_noalloc_forward_refuses_what_it_cannot_serve():
         torch.cuda.synchronize()
         assert torch.equal(y1, y2)
     ctx.close()
+
+
+@pytest.mark.parametrize("kind", ["f32", "tq8"])
+def test_noalloc_forward_beyond_the_slice_partials(kind):
+    """The adapter's slice partials (16 of 1040 x 1024 floats, 68 MB) do not fit the 64 MiB array, h does: the
+    strided GEMM serves the call, off the split kernels by f32 rounding (4096 + 1024 terms)."""
+    import torch
+
+    dev = torch.device("cuda", 0)
+    ctx = rt.Context(0)
+    n, k, t, r = 64, 4096, 1040, 1024
+    make = rt.HipFrozen.f32 if kind == "f32" else rt.HipFrozen.q8_0
+    w = make(O.Rng(1).vec_normal(n * k, 0.02), n, k, ctx=ctx)
+    g = torch.Generator(device=dev).manual_seed(1)
+    x, a, b = (torch.randn(*s, device=dev, generator=g) for s in ((t, k), (r, k), (n, r)))
+    a *= 1.0 / 64
+    b *= 0.01
+    lv = _ffi.RtqLora(r, float(r), a.data_ptr(), b.data_ptr(), 1)
+    y1, y2 = torch.empty(t, n, device=dev), torch.empty(t, n, device=dev)
+    stream = torch.cuda.current_stream().cuda_stream
+    torch.cuda.synchronize()
+    free0 = torch.cuda.mem_get_info(0)[0]
+    ctx.set_timing(True)
+    _ffi.check(_ffi.lib().rtq_linear_forward_noalloc_d(ctx.handle, w.handle, None, ctypes.byref(lv), x.data_ptr(), t, y1.data_ptr(),
+                                                       stream), "rtq_linear_forward_noalloc_d")
+    torch.cuda.synchronize()
+    assert torch.cuda.mem_get_info(0)[0] == free0
+    ran = ctx.timing()
+    ctx.reset_timing()
+    _ffi.check(_ffi.lib().rtq_linear_forward_d(ctx.handle, w.handle, None, ctypes.byref(lv), x.data_ptr(), t, y2.data_ptr(), stream),
+               "rtq_linear_forward_d")
+    torch.cuda.synchronize()
+    assert all(name.startswith("rtq_m_gemm") for name in ran) and not any(name.startswith("rtq_m_gemm") for name in ctx.timing())
+    size = (x.abs() @ (x.new_tensor(np.abs(_dense(w))).T)) + (x.abs() @ a.abs().T) @ b.abs().T
+    assert ((y1 - y2).abs() <= ((k + r) / 2 + 2) * 2.0 ** -24 * size).all()
+    ctx.close()
+
+
+def _dense(w):
+    """The weight's rows, decoded."""
+    out = np.empty((w.out_dim(), w.in_dim()), np.float32)
+    for i in range(w.out_dim()):
+        w.row(i, out[i])
+    return out
