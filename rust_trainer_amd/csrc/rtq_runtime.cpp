@@ -249,7 +249,7 @@ struct rtq_ctx {
   int dense_split = 1;  // trainer-native products on split bf16 MFMAs where they fit (RTQ_DENSE_SPLIT=0: never)
   int gemvq = 1;      // one-launch GEMV for t <= 4 (rtq_gemvq*_*; RTQ_GEMVQ=0: activation kernel + GEMM)
   int gemvq_wpc = 0;  // its waves per CU (RTQ_GEMVQ_WPC; 0: automatic)
-  int fwd_i8 = -1;    // int8-MFMA forwards (rtq_mmi8_*; RTQ_FWD_I8): -1 automatic (Q8_0 weights), 0 never,
+  int fwd_i8 = -1;    // int8-MFMA forwards (rtq_mmi8_*; RTQ_FWD_I8): -1 automatic, 0 never,
                       // 1 every Q4_0 / Q8_0 weight, wherever the 128- or 64-token tiles are chosen
   int64_t t_launches[K_COUNT] = {};
   double t_ms[K_COUNT] = {};
@@ -676,8 +676,8 @@ rtq_status enqueue_backward_dense(rtq_ctx* c, const rtq_weight* w, const float* 
 // of wrg row groups of 16), both of one whole call in us: a launch and its start, then per 1024 columns what a
 // tile takes beside the others on its CU (32-token) or per round of the chip (eight-wave).  Over 1714 calls of 512
 // to 65536 rows, 256 to 9728 columns and 17 to 1000 tokens (profiles/forward_small_grids.md) the choice is the
-// slower one by more than 5% in 7, by 14% at most.  A lower limit of 1.5 tiles per CU took the slower one in a
-// seventh of them, by up to 2.2 times: 8192 x 1024 at 140 tokens 26 us against 17, 40000 x 1024 at 25 33 / 22
+// slower one by more than 5% in 7, by 14% at most.  A limit of 1.5 tiles per CU alone took the slower one in a
+// seventh of them: 8192 x 1024 at 140 tokens 26 us against 17, 40000 x 1024 at 25 33 against 22
 bool fwd_mm32_wins(const rtq_ctx* c, const rtq_weight* w, int64_t mm32, int wrg, int64_t tiles) {
   static const double beside[4] = {8.0, 10.3, 13.1, 18.0}, start[3] = {2.0, 2.8, 4.2}, round[3] = {2.3, 2.6, 3.2};
   const double k = w->cols / 1024.0;
@@ -822,7 +822,9 @@ rtq_status enqueue_forward(rtq_ctx* c, const rtq_weight* w, const float* x, int6
   //      columns: 53565 rows, 384 tokens, 256, 1024 columns 62 / 77, 99 / 108 (at 2048 154 / 158, but 121 / 115 at
   //      256 tokens);
   //    - on rows of 256 columns from one per CU, where the int8 form is up to 16% faster or 27% slower;
-  //  * else 32-token or eight-wave tiles, by the time of each (fwd_mm32_wins).
+  //  * else 32-token tiles where they give 1.5 workgroups per CU, or 64-token ones over tokens padded to 128 one, and
+  //    their time is the lower one (fwd_mm32_wins); else the eight-wave tiles.  (Without the lower limit a small
+  //    model's packed batch and its examples would run on different kernels: their log-probs agree bit for bit.)
   // Measured per forward kernel, us, i8-64 / f16-128 / f16-32 / eight-wave: Q4_0 4096 x 1024 at 256, 512, 1001,
   // 2048 tokens 17 / 23 / 13 / 18, 18 / 24 / 16 / 26, 22 / 26 / 28 / 49, 38 / 36 / 46 / 89; 6144 x 1024 at
   // 1001, 2048 28 / 34 / 36 / 66, 50 / 53 / 66 / 129; 151936 x 1024 at 37, 256, 512 69 / 71 / 91 / 103,
@@ -844,7 +846,7 @@ rtq_status enqueue_forward(rtq_ctx* c, const rtq_weight* w, const float* x, int6
                           (mm128 >= 16 * cu || (mm64 > 3 * cu && mm64 <= 4 * cu && mm128 <= 2 * cu) ||
                            (mm128 >= cu && (w->cols <= 256 || (w->cols <= 1024 && w->rows % 4 && t > 64))));
       if (5 * mm64 >= 8 * cu && (w->rows % 4 == 0 || mm128 >= cu)) mm_ttn = q4_f16 ? 8 : 4;
-      else if (fwd_mm32_wins(c, w, mm32, wrg, gx * gy)) mm_ttn = 2;
+      else if ((2 * mm32 >= 3 * cu || mm_rows * (p.Tp / 64) >= cu) && fwd_mm32_wins(c, w, mm32, wrg, gx * gy)) mm_ttn = 2;
     }
     // a Q4_0 weight's 64-token tiles asked for by RTQ_FWD_MM stay the f16 kernel's
     mmi8 = mm_ttn >= 4 && (c->fwd_i8 == 1 || (c->fwd_i8 < 0 && (w->type == RTQ_TYPE_Q8_0 || (c->fwd_mm < 0 && mm_ttn == 4))));
