@@ -31,13 +31,13 @@
 // of their own (the order the fragments want) held the forward at 0.9 lookups per cycle: 273 us against
 // 230 at 4096 x 4096, 1024 tokens, and 212 without the bank conflicts below.  A fragment (16 rows x 32 elements of one plane) is 64 16-byte
 // slots, row r of k-group g at (r ^ g) + 16 g, a transposed weight tile's fragments lie one slot further
-// apart, and the eight rows of a wave's load are 4 apart (two sets): reads and writes then meet every
-// bank once (a 16-byte access serves lanes 0-3, 12-15, 20-23, 24-27 together, an 8-byte one a half-wave).
-// Measured, TQ8_0 2048 x 1024, 300 tokens, forward + backward with a rank-8 adapter, whole call: 317 us
+// apart, and the eight rows of a wave's load are 4 apart (two sets): reads and writes then spread
+// over the banks (a 16-byte access serves lanes 0-3, 12-15, 20-23, 24-27 together, an 8-byte one a half-wave;
+// conflicts are 0.1% of the forward's cycles and 6% of the backward's).
+// Measured, TQ8_0 2048 x 1024, 300 tokens, forward + backward with a rank-8 adapter, whole call: 313 us
 // on the f32 MFMA GEMM with one launch per adapter product, 61 here (six products: 59; 4096 x 4096, 1024 tokens,
-// backward 327 against 300);
-// against float64 1e-6 there, 2.2e-7 here.  Bound by the wait of each step (one barrier, LDS and MFMA
-// latency) at small grids, by MFMA (38% busy) and LDS (48%) at large ones.
+// backward 327 against 300); against float64 8.5e-7 there, 2.6e-7 here.  Bound by the wait of each step (one
+// barrier, LDS and MFMA latency) at small grids, by MFMA and LDS at large ones.
 #define DENSE_D 4
 constexpr int kDenseFrag = 64;  // 16-byte slots of a fragment
 __device__ __forceinline__ int dense_slot(int r, int g) { return (r ^ g) + 16 * g; }

@@ -290,8 +290,8 @@ __device__ __forceinline__ void lora_load_m(const float* M, int ldm, int r, int 
 // the first rank tile's M values mv (lora_load_m at j0 = 0, loaded by the caller so that they travel with
 // its own loads); each next tile's loads are issued before the current one is contracted.
 // NTOK: tokens t0 .. t0 + NTOK - 1 are written (sx's other rows are zeros).
-// Measured against staging by 16 scalar stores a thread (three LDS cycles in four were conflicts), Q8_0 14336 x
-// 4096, 2048 tokens, r = 64: rtq_act_prep_q8_0 45 -> 33 us (also at 80 VGPRs instead of 184), rtq_bwd_prep 103 -> 88.
+// LDS bank conflicts are 1% of the kernels' cycles.  Measured against staging by 16 scalar stores a thread, Q8_0
+// 14336 x 4096, 2048 tokens, r = 64: rtq_act_prep_q8_0 45 -> 33 us (also at 80 VGPRs instead of 184), rtq_bwd_prep 103 -> 88.
 template <int NTOK = 16>
 __device__ __forceinline__ void lora_partial_v(f4 mv[4], int T, const float* M, int ldm, int r, int k0, int kend, int t0,
                                                float* out, int pstride, int pidx, const f4* sx, f4* sm, float* red) {
@@ -2834,7 +2834,7 @@ extern "C" __global__ __launch_bounds__(256) void rtq_bwd_prep(BwdPrepArgs a) {
 // Bound by its three MFMAs per product at large T: rtq_dxw_q8_0, 14336 x 4096 at 2048 tokens, 783 -> 704 us
 // (1.02 PFLOP/s of f16 MFMA; a library f16 matmul reaches 1.15 here) with eight lanes per dy row instead
 // of one (the L1 looks up a line per cycle: a load of 64 different rows held the kernel to it) and
-// conflict-free LDS; rtq_dxw_q6_k, 2560 x 9728 at 6792 tokens, 1461 -> 1204 us.
+// swizzled LDS (bank conflicts 3 - 6% of its cycles, 14 before); rtq_dxw_q6_k, 2560 x 9728 at 6792 tokens, 1461 -> 1204 us.
 // Three f16 MFMAs per product (dh.wh + dl.wh + dh.wl): the missing dl.wl term and the rounding
 // of dl leave a relative error near 2^-21 per product; the partial is scaled back by 2^-e (exact).
 // Weights whose values could reach 2^15 are pre-scaled by 2^-sigma (wsc) and scaled back in the
@@ -2848,7 +2848,7 @@ extern "C" __global__ __launch_bounds__(256) void rtq_bwd_prep(BwdPrepArgs a) {
 // The converted pair of rows goes to LDS as one 32-bit word per column.  Column k = 32 jb + .. lies at
 // row k ^ jb (its two low bits), its 8-row units XORed with 2 (k / 8 % 2): the words of a half-wave's
 // store (four blocks, eight row pairs) and the 16-byte reads of a fragment (lanes 0-3, 12-15, 20-23,
-// 24-27 are served together) then meet every bank once.
+// 24-27 are served together) then spread over the banks (3 - 6% of the kernel's cycles are conflicts).
 
 template <int FMT, int NQ = 1>
 struct DxSlot {

@@ -675,7 +675,7 @@ rtq_status enqueue_backward_dense(rtq_ctx* c, const rtq_weight* w, const float* 
 // Whether a Q4_0 / Q8_0 forward is faster on 32-token tiles (mm32 of them) than on the eight-wave tiles (`tiles`
 // of wrg row groups of 16), both of one whole call in us: a launch and its start, then per 1024 columns what a
 // tile takes beside the others on its CU (32-token) or per round of the chip (eight-wave).  Over 1714 calls of 512
-// to 65536 rows, 256 to 9728 columns and 17 to 1000 tokens (profiles/forward_small_grids.md) the choice is the
+// to 65536 rows, 256 to 9728 columns and 17 to 1000 tokens the choice is the
 // slower one by more than 5% in 7, by 14% at most.  A limit of 1.5 tiles per CU alone took the slower one in a
 // seventh of them: 8192 x 1024 at 140 tokens 26 us against 17, 40000 x 1024 at 25 33 against 22
 bool fwd_mm32_wins(const rtq_ctx* c, const rtq_weight* w, int64_t mm32, int wrg, int64_t tiles) {
@@ -856,7 +856,7 @@ rtq_status enqueue_forward(rtq_ctx* c, const rtq_weight* w, const float* x, int6
   // K-quants: the LDS-ring kernel from a number of its 128 x 64 tiles (of tokens < t) per CU, else the tile kernel
   // (rtq_fwd_*_w), whose waves split the columns: 0.75 per CU at up to 512 columns, rising to 1.5 (Q4_K; reached at
   // 1102 columns) or 1.75 (Q6_K; 1299).  Measured per call, ring / tile, over 512 to 120000 rows and 17 to 1024
-  // tokens (profiles/forward_small_grids.md), by tiles per CU: 256 columns 0.5 1.05, 0.75 0.77, 1 0.72 - 0.91, 1.5
+  // tokens, by tiles per CU: 256 columns 0.5 1.05, 0.75 0.77, 1 0.72 - 0.91, 1.5
   // 0.67; 512: 0.5 1.1 - 1.18, 0.75 0.93, 1 0.8; 1024, Q4_K: 1 1.02, 1.25 1.06, 1.5 0.95, 2 0.8; Q6_K: 1.25 1.14,
   // 1.5 1.01, 2 0.86; from 2048, Q4_K: 1.25 1.13 - 1.26, 1.5 1.01 - 1.08, 1.75 0.95; Q6_K: 1.5 1.08 - 1.21, 1.75
   // 0.96 - 1.08, 2 0.84 - 0.96.  (One limit of 1.5 had 14148 x 256 at 79 tokens on 14.9 us instead of 10.8.)
@@ -972,10 +972,12 @@ struct DxPlan {
 };
 // The tiles of a t > 16 plan are summed whole in full rounds of the chip (nfull of them; one 256-token
 // workgroup per CU, or two 64-token ones); the rest are split over `splits` workgroups each.  Kind and splits
-// by the time this model gives (us), fitted to the kernels' times over Q4_0 / Q8_0 / Q4_K / Q6_K weights of
-// 3072 x 1024 to 4096 x 14336 at 37 to 2048 tokens (within 15% of 140 measured plans): a 32-row step of a
-// 256-token workgroup 1.6 after 12 of start-up; of a 64-token one 0.65 alone on its CU, 1.0 beside another
-// (K-quants 0.75, 1.15) after 4; each further partial tile (written, read by the finish) 0.05 / 0.02.
+// by the time this model gives (us): a 32-row step of a 256-token workgroup 1.6 after 12 of start-up; of a
+// 64-token one 0.65 alone on its CU, 1.0 beside another (K-quants 0.75, 1.15) after 4; each further partial tile
+// (written, read by the finish) 0.05 / 0.02.  Against 144 measured plans over Q4_0 / Q8_0 / Q4_K / Q6_K weights of 1024
+// to 14336 rows and columns at 17 to 2048 tokens it is 0.7 to 2.5 times the kernel's time (short 256-token plans
+// are overpriced most), but the kind that it takes is the faster one, with its finish, or within 5% of it, in
+// 67 of 72 calls, and 11% slower at worst.
 // Measured, us with the finish, the former rule (64-token tiles unless 256-token ones fill 85% of their
 // rounds) / this one: Q4_K 9728 x 2560 at 37, 256, 1001 tokens 37 / 31, 93 / 61, 337 / 184; Q6_K 2560 x 9728
 // at 100, 1001 53 / 43, 271 / 205; Q8_0 6144 x 4096 at 37 46 / 25
