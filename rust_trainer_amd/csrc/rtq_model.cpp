@@ -1282,7 +1282,7 @@ rtq_status block_backward(rtq_model* m, int l, int64_t t, const float* x, const 
   }
   // every input of the deferred dA / dB (dy, x of each linear, the h / g slots) is still intact here.
   // (Run on a second stream, overlapping the next block's backward, the batch measured slower:
-  // 13.79 against 13.45 ms per configs[2] step - its workgroups hold CUs the next dx kernels need.)
+  // 13.79 against 13.45 ms per 512-token step of the Qwen3-0.6B shape - its workgroups hold CUs the next dx kernels need.)
   if (m->defer_lg)  // every input (dy, x of each linear, the layer's h / g slots) stays intact to the end
     m->lg_all.insert(m->lg_all.end(), jobs.begin(), jobs.end());
   else

@@ -238,7 +238,7 @@ struct rtq_ctx {
   int fwd_waves = 8;  // waves splitting K in the wide Q4_0 / Q8_0 forward (RTQ_FWD_WAVES: 4 or 8)
   int fwd_rg = -1;    // row groups of 16 per eight-wave forward tile: -1 automatic, 1, 2 or 3 (RTQ_FWD_RG)
   int act_tt = 8;     // token tile of the block norms' Q8_0 activation kernel: 16, 8 or 4 (RTQ_ACT_TT;
-                      // configs[2] step, activation kernels: 1.11 / 0.97-1.00 / 1.08 ms)
+                      // 512-token Qwen3-0.6B-shaped step, activation kernels: 1.11 / 0.97-1.00 / 1.08 ms)
   int g64_min = -1;   // fewest 64-token g-partial workgroups (else 16-token ones): -1 = CUs / 2 (RTQ_G64_MIN)
   int fwd_mm = -1;    // large-grid forward: -1 automatic, 0 never, 1 / 2 / 3 the 128- / 64- / 32-token tiles
                       // whenever the format allows (RTQ_FWD_MM)
@@ -546,7 +546,7 @@ const rtq_weight* dense_q8(const rtq_weight* w) { return w->type == RTQ_TYPE_TQ8
 // CU one; else 32 where those give at least half of the CUs one and no CU two (the 32-token
 // form splits each slice's rows over two waves, so twice the workgroups run half the MFMA
 // chain); else 64 where those give at least half of the CUs one; else 16.  Measured per
-// configs[2] call (512 tokens): q|k|v (16 slices, r 48) 8.33 -> 7.46 us at 32; gate|up (24
+// call of the Qwen3-0.6B-shaped step (512 tokens): q|k|v (16 slices, r 48) 8.33 -> 7.46 us at 32; gate|up (24
 // slices, r 32, 384 workgroups at 32) 8.53 -> 9.41, so 64 there
 int prep_gtok(const rtq_ctx* c, int64_t t, int64_t ngq) {
   if (c->gtok == 16 || c->gtok == 32 || c->gtok == 64) return c->gtok;
@@ -673,17 +673,43 @@ rtq_status enqueue_backward_dense(rtq_ctx* c, const rtq_weight* w, const float* 
 }
 
 // Whether a Q4_0 / Q8_0 forward is faster on 32-token tiles (mm32 of them) than on the eight-wave tiles (`tiles`
-// of wrg row groups of 16), both of one whole call in us: a launch and its start, then per 1024 columns what a
-// tile takes beside the others on its CU (32-token) or per round of the chip (eight-wave).  Over 1714 calls of 512
-// to 65536 rows, 256 to 9728 columns and 17 to 1000 tokens the choice is the
-// slower one by more than 5% in 7, by 14% at most.  A limit of 1.5 tiles per CU alone took the slower one in a
-// seventh of them: 8192 x 1024 at 140 tokens 26 us against 17, 40000 x 1024 at 25 33 against 22
-bool fwd_mm32_wins(const rtq_ctx* c, const rtq_weight* w, int64_t mm32, int wrg, int64_t tiles) {
+// of wrg row groups of 16; mm64 tiles of 128 rows x 64 tokens), both of one whole call in us: a launch and its start,
+// then per 1024 columns what a tile takes beside the others on its CU (32-token) or per round of the chip
+// (eight-wave), and what a rank-r adapter costs the eight-wave tiles more (each sums the slices of h for its 64
+// tokens again, 3 to 8 times as many workgroups).  Over 1714 calls of 512 to 65536 rows, 256 to 9728 columns and 17
+// to 1000 tokens without an adapter the choice is the slower one by more than 5% in 7, by 14% at most.  A limit of
+// 1.5 tiles per CU alone took the slower one in a seventh of them: 8192 x 1024 at 140 tokens 26 us against 17, 40000
+// x 1024 at 25 33 against 22
+bool fwd_mm32_wins(const rtq_ctx* c, const rtq_weight* w, int64_t mm32, int64_t mm64, int wrg, int64_t tiles, int64_t r) {
   static const double beside[4] = {8.0, 10.3, 13.1, 18.0}, start[3] = {2.0, 2.8, 4.2}, round[3] = {2.3, 2.6, 3.2};
-  const double k = w->cols / 1024.0;
+  const double k = w->cols / 1024.0, lora = 0.12 * k * r * mm64 / c->cu_count;
   const double one = w->type == RTQ_TYPE_Q4_0 ? 8.4 : beside[0];  // alone on its CU
   const int64_t n = std::min<int64_t>(std::max<int64_t>(cdiv(mm32, c->cu_count), 1), 4);
-  return 6.0 + k * (n == 1 ? one : beside[n - 1]) < 5.0 + cdiv(tiles, c->cu_count) * (start[wrg - 1] + k * round[wrg - 1]);
+  return 6.0 + k * (n == 1 ? one : beside[n - 1]) < 5.0 + cdiv(tiles, c->cu_count) * (start[wrg - 1] + k * round[wrg - 1]) + lora;
+}
+
+// Token tiles of 16 per workgroup of the LDS-ring kernel that a K-quant forward takes (4 or 2; 0: the tile kernel,
+// rtq_fwd_*_w, whose waves split the columns), by its 128 x 64 tiles (of tokens < t) per CU, m, and the adapter's
+// rank, which costs the tile kernel more (its 32-row workgroups sum h's slices four times as often).  Measured per
+// call over 512 to 120000 rows and 17 to 1500 tokens, ring / tile:
+//   no adapter: 256 columns m 0.5 1.05, 0.75 0.77, 1 0.72 - 0.91; 512: 0.5 1.1 - 1.18, 0.75 0.93, 1 0.8; 1024, Q4_K:
+//   1 1.02, 1.25 1.06, 1.5 0.95, 2 0.8, Q6_K: 1.25 1.14, 1.5 1.01, 2 0.86; from 2048, Q4_K: 1.25 1.13 - 1.26, 1.5
+//   1.01 - 1.08, 1.75 0.95, Q6_K: 1.5 1.08 - 1.21, 1.75 0.96 - 1.08, 2 0.84 - 0.96;
+//   rank 16: 1024 columns 0.75 1.04, 1 0.98, 1.5 0.91; 2560 to 9728: 1 1.04 - 1.15, 1.25 1.09 - 1.18, 1.5 0.94 - 1.03;
+//   rank 64: 1024 0.56 1.00, 1 0.91; 2560 to 9728: 0.56 0.93 - 1.13, 0.75 0.88 - 1.10, 1 0.68 - 0.96, 1.5 0.62 - 0.84.
+// 32-token tiles over 64-token ones: up to 32 tokens 0.83 - 0.95; else to m 1.5 without an adapter 0.94 - 1.08, rank 16
+// 0.91 - 1.04 (to 1024 columns 0.98), rank 64 0.82 - 0.99; past it 1.1 - 1.4.  (One limit of 1.5 had 14148 x 256 at 79
+// tokens on 14.9 us instead of 10.8, and with rank 64 4096 x 9728 at 800 on 429 instead of 238.)
+int kquant_ring(const rtq_ctx* c, const rtq_weight* w, int64_t t, int64_t mm64, int64_t r) {
+  const double m = (double)mm64 / c->cu_count;
+  // 0.75 at up to 512 columns, rising to 1.5 (Q4_K, at 1102 columns) or 1.75 (Q6_K, at 1299)
+  double least = std::min(w->type == RTQ_TYPE_Q4_K ? 1.5 : 1.75, 0.75 + 0.65 * (std::max<int64_t>(w->cols, 512) / 512.0 - 1.0));
+  least /= 1.0 + 0.01 * r;
+  if (t <= 32) least = std::min(least, 1.0);
+  const bool wide = r > 16 && m * (12.0 + 0.2 * (r - 16)) >= 11.7;
+  const bool shallow = t > 32 && ((w->cols <= 512 && m > 0.5) || (w->cols <= 256 && m >= 0.375));
+  if (m < least && !wide && !shallow) return 0;
+  return t <= 32 || (m <= 1.5 && (r >= 32 || (r > 0 && w->cols <= 1024))) || (w->cols <= 512 && m < 0.75) ? 2 : 4;
 }
 
 // ------------------------------------------------------------------ enqueue: forward
@@ -812,7 +838,8 @@ rtq_status enqueue_forward(rtq_ctx* c, const rtq_weight* w, const float* x, int6
   const int64_t rg_per_wg = p.skinny ? kFwdSkinnyRG : (w8 ? wrg : wide_rg(w->type));
   const int64_t gx = cdiv(w->Np / 16, rg_per_wg);
   // the large-grid kernels (tiles of 128 rows x 128, 64 or 32 tokens; tokens < t only).  Automatic:
-  //  * the int8-MFMA form on 64-token tiles where those give 1.6 workgroups per CU (on a row count that is no
+  //  * the int8-MFMA form on 64-token tiles where those give 1.6 workgroups per CU (1.73 with a rank-64 adapter, whose
+  //    h the smaller tiles sum as fast: at 1.5 it takes 1.02 of the 32-token tiles' time without one, 1.09 so; on a row count that is no
   //    multiple of 4 where the 128-token tiles give one: Q8_0 30710 x 640, 105 tokens, 32-token tiles 23 us, int8
   //    25); both forms agree bit for bit without an adapter.  Q4_0: the f16 form on 128-token tiles
   //    - from 16 of those per CU;
@@ -845,34 +872,17 @@ rtq_status enqueue_forward(rtq_ctx* c, const rtq_weight* w, const float* x, int6
       const bool q4_f16 = w->type == RTQ_TYPE_Q4_0 &&
                           (mm128 >= 16 * cu || (mm64 > 3 * cu && mm64 <= 4 * cu && mm128 <= 2 * cu) ||
                            (mm128 >= cu && (w->cols <= 256 || (w->cols <= 1024 && w->rows % 4 && t > 64))));
-      if (5 * mm64 >= 8 * cu && (w->rows % 4 == 0 || mm128 >= cu)) mm_ttn = q4_f16 ? 8 : 4;
-      else if ((2 * mm32 >= 3 * cu || mm_rows * (p.Tp / 64) >= cu) && fwd_mm32_wins(c, w, mm32, wrg, gx * gy)) mm_ttn = 2;
+      if (mm64 >= (1.6 + 0.002 * (lora ? r : 0)) * cu && (w->rows % 4 == 0 || mm128 >= cu)) mm_ttn = q4_f16 ? 8 : 4;
+      else if ((2 * mm32 >= 3 * cu || mm_rows * (p.Tp / 64) >= cu) && fwd_mm32_wins(c, w, mm32, mm64, wrg, gx * gy, lora ? r : 0)) mm_ttn = 2;
     }
     // a Q4_0 weight's 64-token tiles asked for by RTQ_FWD_MM stay the f16 kernel's
     mmi8 = mm_ttn >= 4 && (c->fwd_i8 == 1 || (c->fwd_i8 < 0 && (w->type == RTQ_TYPE_Q8_0 || (c->fwd_mm < 0 && mm_ttn == 4))));
     if (mmi8) mm_ttn = 4;
   }
   const bool mm = mm_ttn > 0;
-  // K-quants: the LDS-ring kernel from a number of its 128 x 64 tiles (of tokens < t) per CU, else the tile kernel
-  // (rtq_fwd_*_w), whose waves split the columns: 0.75 per CU at up to 512 columns, rising to 1.5 (Q4_K; reached at
-  // 1102 columns) or 1.75 (Q6_K; 1299).  Measured per call, ring / tile, over 512 to 120000 rows and 17 to 1024
-  // tokens, by tiles per CU: 256 columns 0.5 1.05, 0.75 0.77, 1 0.72 - 0.91, 1.5
-  // 0.67; 512: 0.5 1.1 - 1.18, 0.75 0.93, 1 0.8; 1024, Q4_K: 1 1.02, 1.25 1.06, 1.5 0.95, 2 0.8; Q6_K: 1.25 1.14,
-  // 1.5 1.01, 2 0.86; from 2048, Q4_K: 1.25 1.13 - 1.26, 1.5 1.01 - 1.08, 1.75 0.95; Q6_K: 1.5 1.08 - 1.21, 1.75
-  // 0.96 - 1.08, 2 0.84 - 0.96.  (One limit of 1.5 had 14148 x 256 at 79 tokens on 14.9 us instead of 10.8.)
-  // Its 32-token tiles up to 32 tokens (0.83 - 0.95 of the 64-token ones' time; of the tile kernel's from one per
-  // CU 0.9 - 1.05), and at up to 512 columns above half a 64-token one per CU (0.7 - 1.01 of the tile kernel's)
-  const int64_t mmk_tiles = mm64;
-  const double mmk_min = std::min(w->type == RTQ_TYPE_Q4_K ? 1.5 : 1.75, 0.75 + 0.65 * (std::max<int64_t>(w->cols, 512) / 512.0 - 1.0));
-  int mmk_ttn = 0;  // token tiles of 16 per workgroup of the chosen ring kernel, 0: none
-  if (!p.skinny && !isums && kq) {
-    if (c->fwd_mmk > 0) mmk_ttn = c->fwd_mmk == 2 ? 2 : 4;
-    else if (c->fwd_mmk < 0) {
-      if (t <= 32) mmk_ttn = mmk_tiles >= std::min(mmk_min, 1.0) * c->cu_count ? 2 : 0;
-      else if (mmk_tiles >= mmk_min * c->cu_count) mmk_ttn = 4;
-      else if (w->cols <= 512 && 2 * mmk_tiles > c->cu_count) mmk_ttn = 2;
-    }
-  }
+  int mmk_ttn = 0;  // K-quants: token tiles of 16 per workgroup of the ring kernel, 0: the tile kernel
+  if (!p.skinny && !isums && kq)
+    mmk_ttn = c->fwd_mmk < 0 ? kquant_ring(c, w, t, mm64, lora ? r : 0) : c->fwd_mmk == 0 ? 0 : c->fwd_mmk == 2 ? 2 : 4;
   const int64_t mm_tiles = mm_ttn == 8 ? mm128 : mm_ttn == 4 ? mm64 : mm32;
   // split K across workgroups when the output alone gives too few of them (atomics into a
   // zeroed y); every split keeps at least one half chunk per wave (K-quants: one super-block of
@@ -937,7 +947,7 @@ rtq_status enqueue_forward(rtq_ctx* c, const rtq_weight* w, const float* x, int6
     if (!fa.wq || !fa.wd || !fa.wsb || !fa.xq || !fa.xd || !fa.y || (xbs && !fa.xdh))
       return fail(RTQ_ERR_INVALID, "internal: rtq_mmk_* operand missing");
     return launch(c, (mmk_ttn == 4 ? K_MMK64_Q4_K : K_MMK32_Q4_K) + (w->type == RTQ_TYPE_Q4_K ? 0 : 1),
-                  dim3((unsigned)(mmk_ttn == 4 ? mmk_tiles : mm32)), dim3(256), st, fa,
+                  dim3((unsigned)(mmk_ttn == 4 ? mm64 : mm32)), dim3(256), st, fa,
                   mmk_lds_bytes(w->type, mmk_ttn, mmk_ttn == 4 ? RTQ_MM64_RING : RTQ_MM32_RING));
   }
   if (mm) {

@@ -77,21 +77,30 @@ def test_forward_nan_rows(ctx):
         assert np.array_equal(y[~bad], plain[~bad]), wtype
 
 
-@pytest.mark.parametrize("wtype,n,k,t,kernel", [
-    (O.Q4_0, 8192, 1024, 140, "rtq_mm32_q4_0"), (O.Q8_0, 16384, 512, 20, "rtq_mm32_q8_0"), (O.Q4_0, 2048, 4096, 64, "rtq_fwd_q4_0_w8r1"),
-    (O.Q8_0, 8190, 640, 200, "rtq_mm32_q8_0"), (O.Q4_0, 8192, 512, 1024, "rtq_mm_q4_0"), (O.Q4_0, 8199, 512, 900, "rtq_mm_q4_0"),
-    (O.Q4_0, 8192, 512, 700, "rtq_mmi8_64_q4_0"), (O.Q6_K, 8697, 256, 119, "rtq_mmk32_q6_k"), (O.Q4_K, 16384, 512, 31, "rtq_fwd_q4_k_w"),
-    (O.Q4_K, 24576, 512, 31, "rtq_mmk32_q4_k"), (O.Q4_K, 6144, 256, 256, "rtq_mmk64_q4_k"), (O.Q6_K, 6144, 2048, 448, "rtq_fwd_q6_k_w")])
-def test_default_forward_kernels(wtype, n, k, t, kernel):
+@pytest.mark.parametrize("wtype,n,k,t,r,kernel", [
+    (O.Q4_0, 8192, 1024, 140, 0, "rtq_mm32_q4_0"), (O.Q8_0, 16384, 512, 20, 0, "rtq_mm32_q8_0"),
+    (O.Q4_0, 2048, 4096, 64, 0, "rtq_fwd_q4_0_w8r1"), (O.Q8_0, 8190, 640, 200, 0, "rtq_mm32_q8_0"),
+    (O.Q4_0, 8192, 512, 1024, 0, "rtq_mm_q4_0"), (O.Q4_0, 8199, 512, 900, 0, "rtq_mm_q4_0"),
+    (O.Q4_0, 8192, 512, 700, 0, "rtq_mmi8_64_q4_0"), (O.Q8_0, 3072, 4096, 512, 0, "rtq_fwd_q8_0_w8"),
+    (O.Q8_0, 3072, 4096, 512, 64, "rtq_mm32_q8_0"), (O.Q6_K, 8697, 256, 119, 0, "rtq_mmk32_q6_k"),
+    (O.Q4_K, 16384, 512, 31, 0, "rtq_fwd_q4_k_w"), (O.Q4_K, 24576, 512, 31, 0, "rtq_mmk32_q4_k"),
+    (O.Q4_K, 6144, 256, 256, 16, "rtq_mmk32_q4_k"), (O.Q4_K, 6144, 256, 256, 0, "rtq_mmk64_q4_k"),
+    (O.Q6_K, 6144, 2048, 448, 0, "rtq_fwd_q6_k_w"), (O.Q6_K, 2489, 1024, 430, 16, "rtq_fwd_q6_k_w"),
+    (O.Q6_K, 2489, 1024, 430, 64, "rtq_mmk32_q6_k"), (O.Q6_K, 6144, 1024, 520, 64, "rtq_mmk64_q6_k")])
+def test_default_forward_kernels(wtype, n, k, t, r, kernel):
     """Which kernel the default context takes on both sides of its rules' lines, each against the oracle."""
     c = rt.Context(0)
     blocks = O.quantize(wtype, O.Rng(1).vec_normal(n * k, 0.02).reshape(n, k))
     x = O.Rng(2).vec_normal(t * k, 1.0).reshape(t, k)
-    w = rt.HipFrozen(wtype, blocks, n, k, ctx=c)
+    lin = rt.Linear("default", rt.HipFrozen(wtype, blocks, n, k, ctx=c))
+    want = np.asarray(O.frozen_forward(wtype, blocks, n, k, x, nthreads=8), np.float64).reshape(t, n)
+    if r:
+        a, b = O.Rng(3).vec_normal(r * k, 0.05).reshape(r, k), O.Rng(4).vec_normal(n * r, 0.05).reshape(n, r)
+        lin.lora = rt.Lora(r, 2.0 * r, a, b)
+        want += 2 * (x.astype(np.float64) @ a.T.astype(np.float64)) @ b.T.astype(np.float64)
     c.set_timing(True)
-    y = w.forward(x, t).reshape(t, n)
+    y = lin.forward(x, t).reshape(t, n)
     ran = c.timing()
     c.close()
     assert kernel in ran, ran
-    want = np.asarray(O.frozen_forward(wtype, blocks, n, k, x, nthreads=8), np.float64).reshape(t, n)
     assert np.abs(y - want).max() <= 2e-6 * np.abs(want).max()
