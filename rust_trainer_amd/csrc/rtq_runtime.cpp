@@ -730,6 +730,13 @@ rtq_status enqueue_forward(rtq_ctx* c, const rtq_weight* w, const float* x, int6
   if (t <= 0) return RTQ_OK;
   const bool lora = la && lb && r > 0;
   const RankBlocks rbv = lora && rb ? *rb : RankBlocks{};
+  // ranks that a row's up-projection reads: r, or of a block-diagonal adapter its member's (the rows' mean)
+  int64_t up_rank = lora ? r : 0;
+  if (rbv.nm > 0) {
+    up_rank = 0;
+    for (int i = 0; i < rbv.nm; i++) up_rank += (int64_t)rbv.nrow[i] * rbv.r[i];
+    up_rank = cdiv(up_rank, w->rows);
+  }
   if (is_dense(w->type)) {
     if (sw || nf) return fail(RTQ_ERR_UNSUPPORTED, "internal: SwiGLU / norm input of a dense weight");
     return enqueue_forward_dense(c, w, x, t, y, bias, la, lb, lora ? r : 0, s, ar, st);
@@ -872,8 +879,8 @@ rtq_status enqueue_forward(rtq_ctx* c, const rtq_weight* w, const float* x, int6
       const bool q4_f16 = w->type == RTQ_TYPE_Q4_0 &&
                           (mm128 >= 16 * cu || (mm64 > 3 * cu && mm64 <= 4 * cu && mm128 <= 2 * cu) ||
                            (mm128 >= cu && (w->cols <= 256 || (w->cols <= 1024 && w->rows % 4 && t > 64))));
-      if (mm64 >= (1.6 + 0.002 * (lora ? r : 0)) * cu && (w->rows % 4 == 0 || mm128 >= cu)) mm_ttn = q4_f16 ? 8 : 4;
-      else if ((2 * mm32 >= 3 * cu || mm_rows * (p.Tp / 64) >= cu) && fwd_mm32_wins(c, w, mm32, mm64, wrg, gx * gy, lora ? r : 0)) mm_ttn = 2;
+      if (mm64 >= (1.6 + 0.002 * up_rank) * cu && (w->rows % 4 == 0 || mm128 >= cu)) mm_ttn = q4_f16 ? 8 : 4;
+      else if ((2 * mm32 >= 3 * cu || mm_rows * (p.Tp / 64) >= cu) && fwd_mm32_wins(c, w, mm32, mm64, wrg, gx * gy, up_rank)) mm_ttn = 2;
     }
     // a Q4_0 weight's 64-token tiles asked for by RTQ_FWD_MM stay the f16 kernel's
     mmi8 = mm_ttn >= 4 && (c->fwd_i8 == 1 || (c->fwd_i8 < 0 && (w->type == RTQ_TYPE_Q8_0 || (c->fwd_mm < 0 && mm_ttn == 4))));
@@ -882,7 +889,7 @@ rtq_status enqueue_forward(rtq_ctx* c, const rtq_weight* w, const float* x, int6
   const bool mm = mm_ttn > 0;
   int mmk_ttn = 0;  // K-quants: token tiles of 16 per workgroup of the ring kernel, 0: the tile kernel
   if (!p.skinny && !isums && kq)
-    mmk_ttn = c->fwd_mmk < 0 ? kquant_ring(c, w, t, mm64, lora ? r : 0) : c->fwd_mmk == 0 ? 0 : c->fwd_mmk == 2 ? 2 : 4;
+    mmk_ttn = c->fwd_mmk < 0 ? kquant_ring(c, w, t, mm64, up_rank) : c->fwd_mmk == 0 ? 0 : c->fwd_mmk == 2 ? 2 : 4;
   const int64_t mm_tiles = mm_ttn == 8 ? mm128 : mm_ttn == 4 ? mm64 : mm32;
   // split K across workgroups when the output alone gives too few of them (atomics into a
   // zeroed y); every split keeps at least one half chunk per wave (K-quants: one super-block of
