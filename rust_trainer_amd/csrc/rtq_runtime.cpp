@@ -846,9 +846,9 @@ rtq_status enqueue_forward(rtq_ctx* c, const rtq_weight* w, const float* x, int6
   const int64_t gx = cdiv(w->Np / 16, rg_per_wg);
   // the large-grid kernels (tiles of 128 rows x 128, 64 or 32 tokens; tokens < t only).  Automatic:
   //  * the int8-MFMA form on 64-token tiles where those give 1.6 workgroups per CU (1.73 with a rank-64 adapter, whose
-  //    h the smaller tiles sum as fast: at 1.5 it takes 1.02 of the 32-token tiles' time without one, 1.09 so; on a row count that is no
-  //    multiple of 4 where the 128-token tiles give one: Q8_0 30710 x 640, 105 tokens, 32-token tiles 23 us, int8
-  //    25); both forms agree bit for bit without an adapter.  Q4_0: the f16 form on 128-token tiles
+  //    h the smaller tiles sum as fast: at 1.5 it takes 1.02 of the 32-token tiles' time without one, 1.09 so; on a
+  //    row count that is no multiple of 4 where the 128-token tiles give one: Q8_0 30710 x 640, 105 tokens, 32-token
+  //    tiles 23 us, int8 25); both forms agree bit for bit without an adapter.  Q4_0: the f16 form on 128-token tiles
   //    - from 16 of those per CU;
   //    - where they need one round of the chip (two a CU) and the int8 ones, three a CU, a second: 8192 x 1024 at
   //      1024 tokens 39 / 40 us, 28672 x 1024 at 256 35 / 37, 14336 x 256 at 512 18 / 20;
